@@ -29,6 +29,9 @@ enum AMode : int {
                  // for A_CONVP when the window fits and conv_window is set
 };
 
+// Width of the GPT decoder's residual stream (EPI_KVCACHE's column sections).
+constexpr int kGptW = 1280;
+
 // A_CONVW: LDS halves of a BM-row block's input window.  The window holds
 // rows m0 - conv_pad .. m0 + BM - 1 + (conv_k - 1) conv_d - conv_pad of the
 // operand, each padded to conv_window_chunks(conv_c) 16-byte chunks (the
@@ -57,6 +60,10 @@ enum EpiMode : int {
   EPI_DUAL = 7,       // cols < N/2 -> C32 (+ f16 copy C16); cols >= N/2 -> C32b
   EPI_RESAVG = 8,     // v = acc + bias + res; C32 = v (optional); g = (flag ? C32b : 0) + v / 3
                       // -> C32b, and its f16 copy -> C16 (optional)
+  EPI_GELU16 = 9,     // C16 (+ its lo half at c16_lo) = gelu_new(acc + bias)
+  EPI_KVCACHE = 10,   // N = 3 x kGptW, v = acc + bias: columns < kGptW -> C32; the next kGptW
+                      // -> C32b and the rest -> C32c, the head-major caches
+                      // [head][Tpad rows][64], at cache row T + m
 };
 
 struct GemmArgs {
@@ -91,6 +98,8 @@ struct GemmArgs {
   int ldc16 = 0;
   float* C32b = nullptr;
   int ldc32b = 0;
+  float* C32c = nullptr;             // EPI_KVCACHE: the value cache
+  int* overflow = nullptr;           // EPI_GELU16: set to 1 when an output does not fit f16
   const float* cond = nullptr;       // EPI_GATE: [a(512) | b(512)] global conditioning
   const uint32_t* mask = nullptr;    // per-row 0/1 (WaveNet epilogues)
   const float* rp = nullptr;         // EPI_FINALSKIP: res_projection [M][512]
@@ -190,11 +199,26 @@ __device__ inline void split_f16(float v, half_t& hi, half_t& lo) {
   lo = (half_t)((v - (float)hi) * kSplitScale);
 }
 
+// Largest magnitude a split pair holds (its hi half is finite).
+constexpr float kSplitMax = 65504.0f;
+
+// cpu_gelu_new (tokenizer_tests.cpp:3931-3945)
+__device__ __forceinline__ float gelu_new(float v) {
+  if (v > 10.0f) return v;
+  if (v < -10.0f) return 0.0f;
+  return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+}
+
 // Number of per-row partial sums of squares a 512-wide producer writes.
 constexpr int kSsqParts = 16;
 
 // Picks a tile shape for (M, N) and launches; returns hipSuccess or the
 // launch error.  Host-side checks reject shapes the kernels do not cover.
 hipError_t launch_gemm(const GemmArgs& a, AMode amode, EpiMode epi, hipStream_t stream);
+
+// The GPT prefill's products: A_PLAIN with a split A and an f16-exact W
+// (GemmArgs::split = 1), epilogue EPI_KVCACHE, EPI_GELU16 or EPI_F32 (with a
+// residual).  K a multiple of 256, N of 64.
+hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream);
 
 }  // namespace mit2hip

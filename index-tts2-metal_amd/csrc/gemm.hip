@@ -587,6 +587,17 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
       for (int j = 0; j < NI; ++j) accx[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
+  // The GPT prefill's long sums: each stage's product is summed by itself and
+  // then added to the total, so no value passes through a chain of K / 32
+  // matrix-core additions.
+  constexpr bool kFold = AM == A_PLAIN && SP == 1;
+  floatx4 tot[kFold ? MI : 1][kFold ? NI : 1];
+  if constexpr (kFold) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) tot[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // Fragment reads.  Every fragment row of this lane has the same swizzle
   // (rows differ by multiples of 16), so a read's address is the stage
@@ -654,6 +665,15 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
           for (int j = 0; j < NI; ++j) accx[i][j] = mfma16x16x32(bfl[j], af[i], accx[i][j]);
       }
+    }
+    if constexpr (kFold) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
     }
   };
 
@@ -843,6 +863,12 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
       for (int j = 0; j < NI; ++j) acc[i][j] += acc1[i][j];  // part 0 + part 1
   }
+  if constexpr (kFold) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j];
+  }
   if constexpr (SP > 0) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -932,7 +958,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
                                                       nsa[j].z * nsg[j].z, nsa[j].w * nsg[j].w);
   }
   if constexpr (EPI == EPI_F32 || EPI == EPI_F16 || EPI == EPI_DUAL || EPI == EPI_RESSKIP ||
-                EPI == EPI_FINALSKIP || EPI == EPI_RESAVG) {
+                EPI == EPI_FINALSKIP || EPI == EPI_RESAVG || EPI == EPI_GELU16 || EPI == EPI_KVCACHE) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       const int m = row_base + 16 * i;
@@ -1002,6 +1028,21 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
         if (!live) continue;
         if constexpr (EPI == EPI_F16) {
           st16s(p.C16 + (size_t)m * p.ldc16 + n, v.x, v.y, v.z, v.w);
+        } else if constexpr (EPI == EPI_GELU16) {
+          const float4 y = make_float4(gelu_new(v.x), gelu_new(v.y), gelu_new(v.z), gelu_new(v.w));
+          // (written so that a NaN counts as not fitting)
+          if (!(fabsf(y.x) <= kSplitMax && fabsf(y.y) <= kSplitMax && fabsf(y.z) <= kSplitMax &&
+                fabsf(y.w) <= kSplitMax))
+            *p.overflow = 1;
+          st16s(p.C16 + (size_t)m * p.ldc16 + n, y.x, y.y, y.z, y.w);
+        } else if constexpr (EPI == EPI_KVCACHE) {
+          if (n < kGptW) {
+            *reinterpret_cast<float4*>(p.C32 + (size_t)m * p.ldc32 + n) = v;
+          } else {  // four columns of one head (64-column heads, n a multiple of 4)
+            const int c = n - (n < 2 * kGptW ? kGptW : 2 * kGptW);
+            float* cache = n < 2 * kGptW ? p.C32b : p.C32c;
+            *reinterpret_cast<float4*>(cache + ((size_t)(c >> 6) * p.Tpad + p.T + m) * 64 + (c & 63)) = v;
+          }
         } else if constexpr (EPI == EPI_DUAL) {
           const int half_n = p.N >> 1;
           if (n < half_n) {
@@ -1851,6 +1892,44 @@ hipError_t launch_gemm(const GemmArgs& a, AMode amode, EpiMode epi, hipStream_t 
     if (epi == EPI_F32) return launch_am_epi<A_CONV3Z, EPI_F32>(a, stream);
   }
   return hipErrorInvalidValue;  // combination not built
+}
+
+// GPT prefill products (split A, W exact in f16; layer shapes N x K 3840 x
+// 1280, 1280 x 1280, 5120 x 1280 and 1280 x 5120).  A few hundred rows make a
+// few hundred tiles at most, whose time is the latency of their K stages (the
+// weights come from HBM, once): so the tile is the largest that still gives
+// most CUs one, and the ring as deep as the LDS then allows.  Swept over
+// prefixes of 16, 64, 213, 450 and 640 rows (us of a whole 24-layer call with
+// one product's tile changed):
+//  * more than 256 64 x 64 tiles: three stages, so that two workgroups share
+//    a CU (c_fc at 213 rows, 320 tiles: 2149 against 2224 with four stages);
+//  * 129 to 256: four stages (mlp c_proj at 640 rows, 200 tiles: 3708 against
+//    3868 with three);
+//  * at most 160 tiles of 32 x 32 (every product at 16 rows): those, K split
+//    over four wave groups (mlp c_proj at 64 rows: 1697 against 1833 with
+//    32 x 64 tiles and two groups, 2166 with 64 x 64);
+//  * between: 64 x 32 with two groups for the long K (2185 at 213 rows against
+//    2245 with the next), 32 x 64 with five stages for the others (c_fc at 64
+//    rows: 1782 against 1872 with 64 x 64, 1947 with 64 x 32).
+template <int EPI>
+static hipError_t launch_rows_epi(const GemmArgs& a, hipStream_t s) {
+  const long t64 = tile_count(a, 64, 64);
+  if (t64 > 256) return launch_tile<64, 64, 64, 3, A_PLAIN, EPI, 4, 2, 1, 1>(a, s);
+  if (t64 > 128) return launch_tile<64, 64, 64, 4, A_PLAIN, EPI, 4, 2, 1, 1>(a, s);
+  if (tile_count(a, 32, 32) <= 160) return launch_tile<32, 32, 64, 3, A_PLAIN, EPI, 2, 1, 4, 1>(a, s);
+  if (EPI == EPI_F32 && a.K >= 2560) return launch_tile<64, 32, 64, 3, A_PLAIN, EPI, 4, 1, 2, 1>(a, s);
+  return launch_tile<32, 64, 64, 5, A_PLAIN, EPI, 2, 2, 1, 1>(a, s);
+}
+
+hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream) {
+  if (!gemm_spans_fit(a, A_PLAIN) || a.split != 1 || a.a_lo == 0 || !a.A || !a.W || !a.bias || a.K % 256 != 0 ||
+      a.N % 64 != 0 || a.row_nb != 0 || a.n_store != 0 || a.colperm || a.lda < a.K || a.ldw < a.K)
+    return hipErrorInvalidValue;
+  if (epi == EPI_KVCACHE && a.N == 3 * kGptW && a.C32 && a.C32b && a.C32c && a.T >= 0 && a.T + a.M <= a.Tpad)
+    return launch_rows_epi<EPI_KVCACHE>(a, stream);
+  if (epi == EPI_GELU16 && a.C16 && a.c16_lo && a.overflow) return launch_rows_epi<EPI_GELU16>(a, stream);
+  if (epi == EPI_F32 && a.C32) return launch_rows_epi<EPI_F32>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace mit2hip

@@ -19,6 +19,12 @@
 //              c_proj   x += W_mp f + b          (the last layer advances kv)
 //   head       logits = W_head LN_fn(LN_f(x)) + b, argmax, token bookkeeping
 //
+// The prefix goes through the layers before that, all its rows together as
+// matrix-core products (Impl::enqueue_rows, gpt_prefill.hip).  A prefix of 213
+// rows and one more took 40.6 ms as chunks of 8 rows on the vector units
+// (27 passes over the weights) and takes 2.17 ms so; 0.2 ms is what reading the
+// weights once costs, the rest the latency of 24 x 7 dependent launches.
+//
 // Every matrix-vector product is HBM-bound: each weight is read once per
 // step (f16, 0.98 GB for 24 layers) and used for one multiply-add.  The GEMV
 // kernel loads the input vector, then streams whole rows into registers
@@ -41,6 +47,8 @@
 
 #include "device_common.h"
 #include "engine.h"
+#include "gemm.h"
+#include "gpt_prefill.h"
 #include "image_io.h"
 
 namespace mit2hip {
@@ -55,7 +63,7 @@ namespace mit2hip {
 
 namespace {
 
-constexpr int kW = 1280, kQKV = 3840, kMLP = 5120, kHeads = 20, kHD = 64;
+constexpr int kW = kGptW, kQKV = 3840, kMLP = 5120, kHeads = 20, kHD = 64;
 constexpr int kVocab = GptDecoder::kVocab, kPos = GptDecoder::kPositions;
 constexpr int kStart = (int)GptDecoder::kStartToken, kStop = (int)GptDecoder::kStopToken;
 #ifndef GPT_ATTN_KEYS
@@ -64,7 +72,7 @@ constexpr int kStart = (int)GptDecoder::kStartToken, kStop = (int)GptDecoder::kS
 constexpr int kChunk = GPT_ATTN_KEYS;  // keys per attention split
 static_assert(kChunk % 64 == 0 && kChunk <= 512, "a split is whole passes of 64 keys, one score per thread");
 constexpr int kStepsPerCheck = 8;  // decode steps replayed between stop-flag reads
-constexpr int kPrefillRows = 8;    // prefix rows per prefill chunk
+constexpr int kPrefillRows = 1024;  // most prefix rows per prefill chunk (36 KB of workspace a row)
 
 // Device-side decode state.
 struct GptState {
@@ -80,7 +88,7 @@ struct GptState {
   int32_t max_pred;   // capacity of the predicted array (inputs: + 1)
   int32_t cap;        // rows of each key/value cache
   int32_t rows;       // rows of the prefix buffer
-  int32_t pend;       // prefix rows the prefill chunks cover (rows 0..pend-1)
+  int32_t overflow;   // 1: a prefill value did not fit a split f16 pair
   int32_t top_k;      // sampling (sample_kernel): top-k (0: off)
   float temperature;  //   temperature, top-p, repetition penalty
   float top_p;
@@ -117,13 +125,6 @@ struct GemvArgs {
   float* lnf_out = nullptr;   // LOGITS: block 0 writes the two LayerNorm outputs
   float* fn_out = nullptr;
 };
-
-__device__ __forceinline__ float gelu_new(float v) {
-  // cpu_gelu_new (tokenizer_tests.cpp:3931-3945)
-  if (v > 10.0f) return v;
-  if (v < -10.0f) return 0.0f;
-  return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
-}
 
 // Sum over the LPR lanes of a lane group (every lane gets the sum).
 template <int LPR>
@@ -311,113 +312,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
       a.blk_val[blockIdx.x] = bv;
       a.blk_idx[blockIdx.x] = bi;
     }
-  }
-}
-
-// The prefill's multi-row form of gemv_kernel: y[m] = W pro(x[m]) + b for the
-// rows m < mrows = min(kPrefillRows, pend - kv) of a prefix chunk (rows kv..),
-// so each weight row is read once per chunk instead of once per prefix row.
-// The chunk's inputs (normalised first, for the LayerNorm prologue) are
-// staged in LDS; every sum runs in gemv_kernel's order (the same lane
-// layout, the same two partial sums, the same group reduction and the same
-// LayerNorm statistics), so a prefix row gets the same values either way.
-template <int K, int LPR, int WAVES, int PRO, int EPI>
-__global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
-  constexpr int MR = kPrefillRows;
-  constexpr int RPW = 64 / LPR;
-  constexpr int CH = K / (8 * LPR);
-  constexpr int ROWS = WAVES * RPW;
-  static_assert(K % (8 * LPR) == 0, "K must be a multiple of 8 * LPR");
-  static_assert(PRO != PRO_LN2 && EPI != EPI_LOGITS, "the prefill has no head");
-  static_assert(PRO == PRO_PLAIN || K == kW, "LayerNorm prologues take the 1280-wide stream");
-  __shared__ float4 xs[MR][K / 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane / LPR, j = lane % LPR;
-  const int kv = a.st->kv;
-  const int mrows = min(MR, a.st->pend - kv);
-  const int r = blockIdx.x * ROWS + wave * RPW + sub;
-
-  half8 w[CH];
-  {
-    const half8* src = reinterpret_cast<const half8*>(a.w + (size_t)min(r, a.N - 1) * K) + j;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) w[c] = src[c * LPR];
-  }
-  __builtin_amdgcn_sched_barrier(0);
-
-  // stage the chunk's inputs (rows past mrows are zeros)
-  if constexpr (PRO == PRO_PLAIN) {
-    for (int i = threadIdx.x; i < MR * (K / 4); i += WAVES * 64) {
-      const int mm = i / (K / 4), k4 = i % (K / 4);
-      xs[mm][k4] = mm < mrows ? reinterpret_cast<const float4*>(a.x + (size_t)mm * K)[k4]
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  } else {
-    // one wave per row, lanes laid out as a 32-lane group (both halves
-    // compute the same values; the first half stores them)
-    constexpr int CH32 = K / (8 * 32);
-    const int jj = lane & 31;
-    for (int mm = wave; mm < MR; mm += WAVES) {
-      float v[CH32][8];
-      if (mm < mrows) {
-        float g[CH32][8], b[CH32][8];
-        load_chunks<32, CH32>(v, a.x + (size_t)mm * K, jj);
-        load_chunks<32, CH32>(g, a.g1, jj);
-        load_chunks<32, CH32>(b, a.b1, jj);
-        group_layernorm<32, CH32>(v, g, b);
-      } else {
-#pragma unroll
-        for (int c = 0; c < CH32; ++c)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[c][e] = 0.f;
-      }
-      if (lane < 32) {
-#pragma unroll
-        for (int c = 0; c < CH32; ++c) {
-          xs[mm][2 * (jj + 32 * c)] = make_float4(v[c][0], v[c][1], v[c][2], v[c][3]);
-          xs[mm][2 * (jj + 32 * c) + 1] = make_float4(v[c][4], v[c][5], v[c][6], v[c][7]);
-        }
-      }
-    }
-  }
-  __syncthreads();
-
-  float wf[CH][8];
-#pragma unroll
-  for (int c = 0; c < CH; ++c)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) wf[c][e] = (float)w[c][e];
-  // one chunk row at a time (hoisting every row's LDS reads costs registers)
-#pragma unroll
-  for (int mm = 0; mm < MR; ++mm) {
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int q4 = 2 * (j + c * LPR);
-      const float4 lo = xs[mm][q4], hi = xs[mm][q4 + 1];
-      s0 += wf[c][0] * lo.x; s1 += wf[c][1] * lo.y;
-      s0 += wf[c][2] * lo.z; s1 += wf[c][3] * lo.w;
-      s0 += wf[c][4] * hi.x; s1 += wf[c][5] * hi.y;
-      s0 += wf[c][6] * hi.z; s1 += wf[c][7] * hi.w;
-    }
-    const float acc = group_sum<LPR>(s0 + s1);
-    if (j == 0 && r < a.N && mm < mrows) {
-      const float v = acc + a.bias[r];
-      if constexpr (EPI == EPI_GELU) {
-        a.y[(size_t)mm * a.N + r] = gelu_new(v);
-      } else if constexpr (EPI == EPI_RES) {
-        a.y[(size_t)mm * a.N + r] += v;
-      } else {
-        if (r < kW) {
-          a.q[(size_t)mm * kW + r] = v;
-        } else if (kv + mm < a.st->cap) {
-          const int c = r - (r < 2 * kW ? kW : 2 * kW);  // head c / 64, dim c % 64
-          float* cache = r < 2 * kW ? a.kc : a.vc;
-          cache[((size_t)(c >> 6) * a.st->cap + kv + mm) * kHD + (c & 63)] = v;
-        }
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -776,18 +670,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
   st->step += 1;
 }
 
-// Rows kv .. kv + mrows - 1 of the prefix into the chunk buffer.
-__global__ __launch_bounds__(256) void embed_rows_kernel(const GptState* st, const float* rows, float* x) {
-  const int mrows = min(kPrefillRows, st->pend - st->kv);
-  const float4* src = reinterpret_cast<const float4*>(rows + (size_t)st->kv * kW);
-  for (int i = threadIdx.x; i < mrows * (kW / 4); i += 256) reinterpret_cast<float4*>(x)[i] = src[i];
-}
-
-// The chunk is done: its rows join the caches.
-__global__ void advance_rows_kernel(GptState* st) {
-  st->kv += max(0, min(kPrefillRows, st->pend - st->kv));
-}
-
 // argmax_row (gpt.cpp:1297-1308), second stage: the first maximum over the
 // head blocks' maxima (ties go to the lower row), then the bookkeeping of the
 // loop of run_gpt_kv_greedy_cpu (gpt.cpp:1890-1909): record the prediction,
@@ -866,32 +748,30 @@ __global__ __launch_bounds__(320) void embed_kernel(const GptState* st, const fl
 // gpt.cpp:1147-1170, with cpu_attention_single_query, tokenizer_tests.cpp:
 // 4034-4060) over the st->kv + 1 cache rows (the current row included: the
 // c_attn kernel already wrote it), in two launches with no waiting between
-// blocks.  attn_split_kernel: block (head h, split s, query row z) takes keys
+// blocks.  attn_split_kernel: block (head h, split s) takes keys
 // 256 s .. 256 s + 255 -- all of its key and value loads issued together
 // (the kernel is latency-bound) -- and writes the split's max m_s, sum
 // l_s = sum exp(score - m_s) and unnormalised output sum exp(score - m_s) v;
 // a head with a single split writes its output directly.  attn_combine_kernel
 // merges the splits: out = sum_s e^(m_s - M) o_s / sum_s e^(m_s - M) l_s with
 // M = max m_s (eight splits per round trip, rescaled when M grows).  Scores: 8 lanes per key, 8 dims each; the output: 16 lanes
-// per key, 4 dims each.  z is the query row of a prefill chunk (row z sees
-// the keys up to its own position kv + z); a decode step has one query.
+// per key, 4 dims each.
 constexpr int kAttnThreads = 512;
 constexpr int kPartF = 2 + kHD;  // per split: max, sum, unnormalised output
 
 // What an attention block needs from the state: whether it has nothing to do
-// (the decode stopped, row z is past the prefill chunk, or the caches have
-// no rows) and row z's key count.  The four fields are read before anything
-// is decided, and all of them decide, so the loads are issued together and
-// their latencies overlap; tested one after another (as short-circuit tests
-// with the key count read after them), each load waited for the one before.
+// (the decode stopped, or the caches have no rows) and its key count.  The
+// three fields are read before anything is decided, and all of them decide,
+// so the loads are issued together and their latencies overlap; tested one
+// after another (as short-circuit tests with the key count read after them),
+// each load waited for the one before.
 struct AttnRow {
   bool idle;
   int keys;
 };
-__device__ __forceinline__ AttnRow attn_row(const GptState* st, int z, int check_stop) {
-  const int kv = st->kv, stopped = st->stopped, cap = st->cap, pend = st->pend;
-  const bool live = gridDim.z == 1 || z < min((int)gridDim.z, pend - kv);
-  return {(check_stop && stopped) || !live || cap <= 0, min(kv + z + 1, cap)};
+__device__ __forceinline__ AttnRow attn_row(const GptState* st, int check_stop) {
+  const int kv = st->kv, stopped = st->stopped, cap = st->cap;
+  return {(check_stop && stopped) || cap <= 0, min(kv + 1, cap)};
 }
 
 __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q, const float* kc, const float* vc,
@@ -901,13 +781,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
   constexpr int kKeysPerPass = kAttnThreads / 8, kPass = kChunk / kKeysPerPass;
   constexpr int kVKeysPerPass = kAttnThreads / 16, kVPass = kChunk / kVKeysPerPass;
   constexpr int kGroups = kAttnThreads / 16;  // output key groups
-  const int h = blockIdx.x, sp = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
-  const AttnRow row = attn_row(st, z, check_stop);
+  const int h = blockIdx.x, sp = blockIdx.y, tid = threadIdx.x;
+  const AttnRow row = attn_row(st, check_stop);
   if (row.idle) return;
   const int kvn = row.keys;
   const int nsplit = (kvn + kChunk - 1) / kChunk;
   if (sp >= nsplit) return;
-  q += (size_t)z * kW;
   const int t0 = sp * kChunk, n = min(kChunk, kvn - t0), last = kvn - 1;
   __shared__ float sc[kChunk];
   __shared__ float4 red[kGroups][kHD / 4];
@@ -973,9 +852,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
 #pragma unroll
     for (int gg = 0; gg < kGroups; ++gg) od += reinterpret_cast<const float*>(&red[gg][0])[tid];
     if (nsplit == 1) {
-      out[(size_t)z * kW + h * kHD + tid] = od / l;
+      out[h * kHD + tid] = od / l;
     } else {
-      float* pp = part + (((size_t)z * kHeads + h) * nsplit_max + sp) * kPartF;
+      float* pp = part + ((size_t)h * nsplit_max + sp) * kPartF;
       pp[2 + tid] = od;
       if (tid == 0) { pp[0] = m; pp[1] = l; }
     }
@@ -984,12 +863,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
 
 __global__ __launch_bounds__(64) void attn_combine_kernel(const GptState* st, const float* part, float* out,
                                                           int nsplit_max, int check_stop) {
-  const int h = blockIdx.x, z = blockIdx.z, d = threadIdx.x;
-  const AttnRow row = attn_row(st, z, check_stop);
+  const int h = blockIdx.x, d = threadIdx.x;
+  const AttnRow row = attn_row(st, check_stop);
   if (row.idle) return;
   const int nsplit = (row.keys + kChunk - 1) / kChunk;
   if (nsplit == 1) return;  // written by the split kernel
-  const float* ph = part + ((size_t)z * kHeads + h) * nsplit_max * kPartF;
+  const float* ph = part + (size_t)h * nsplit_max * kPartF;
   // eight splits per round trip (the loads are issued before they are used)
   float M = -INFINITY, L = 0.f, O = 0.f;
   for (int s0 = 0; s0 < nsplit; s0 += 8) {
@@ -1018,7 +897,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const GptState* st, co
     }
     M = Mn;
   }
-  out[(size_t)z * kW + h * kHD + d] = O / L;
+  out[h * kHD + d] = O / L;
 }
 
 // Launch shapes: rows per block = WAVES * (64 / LPR) * UR.
@@ -1061,14 +940,6 @@ void launch_fc(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_FC_SHAPE,
 void launch_mlp_proj(const GemvArgs& a, hipStream_t s) { launch_gemv<kMLP, GPT_MP_SHAPE, PRO_PLAIN, EPI_RES>(a, s); }
 void launch_head(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_HEAD_SHAPE, PRO_LN2, EPI_LOGITS>(a, s); }
 
-// The prefill chunk's GEMVs (lanes per row, waves per block).
-template <int K, int LPR, int WAVES, int PRO, int EPI>
-void launch_rows(const GemvArgs& a, hipStream_t s) {
-  constexpr int rows = WAVES * (64 / LPR);
-  hipLaunchKernelGGL((gemv_rows_kernel<K, LPR, WAVES, PRO, EPI>), dim3((a.N + rows - 1) / rows), dim3(WAVES * 64), 0,
-                     s, a);
-}
-
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 }  // namespace
@@ -1095,26 +966,26 @@ struct GptDecoder::Impl {
   GptState* st = nullptr;
   uint32_t *predicted = nullptr, *inputs = nullptr;
   float *x, *q, *att, *fc, *logits, *lnf, *fn, *blk_val, *kc, *vc, *rows;
-  float *xr, *qr, *attr, *fcr;  // a prefill chunk's rows: [8][1280] x3, [8][5120]
+  int chunk_cap = 0;            // rows of the prefill chunk buffers
+  float *xr, *qr;               // a prefill chunk's rows: the residual stream and the queries
+  half_t *a16, *fc16;           //   the products' split operands [2][rows][1280] and [2][rows][5120]
   float* proc = nullptr;        // the sampler's processed logits [8194]
   uint32_t* hist = nullptr;     // the repetition-history prefix [kMaxHistory]
-  float* part = nullptr;        // attention splits: [8 query rows][20 heads][nsplit_max][66]
+  float* part = nullptr;        // attention splits: [20 heads][nsplit_max][66]
   int nsplit_max = 0;
 
   // check_stop: the launch does nothing once the stop token was predicted
   // (decode steps; the timing hook passes 0).
-  void launch_attention(const float* qv, const float* K, const float* V, float* out, int rows_z,
-                        int check_stop = 1) {
-    hipLaunchKernelGGL(attn_split_kernel, dim3(kHeads, nsplit_max, rows_z), dim3(kAttnThreads), 0, s, qv, K, V, st,
-                       part, out, nsplit_max, check_stop);
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(kHeads, 1, rows_z), dim3(kHD), 0, s, st, part, out, nsplit_max,
-                       check_stop);
+  void launch_attention(const float* qv, const float* K, const float* V, float* out, int check_stop = 1) {
+    hipLaunchKernelGGL(attn_split_kernel, dim3(kHeads, nsplit_max), dim3(kAttnThreads), 0, s, qv, K, V, st, part, out,
+                       nsplit_max, check_stop);
+    hipLaunchKernelGGL(attn_combine_kernel, dim3(kHeads), dim3(kHD), 0, s, st, part, out, nsplit_max, check_stop);
   }
   int* blk_idx;
   GptState* host_state = nullptr;  // pinned
-  // row, row + head, token + head, prefill chunk, kStepsPerCheck token steps,
-  // then the sampled forms of the last two token graphs
-  hipGraphExec_t graph[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  // row, row + head, token + head, kStepsPerCheck token steps, then the
+  // sampled forms of the last two token graphs
+  hipGraphExec_t graph[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   bool use_graph = true;  // env MIT2CFM_GRAPH=0: launch every kernel directly (for profilers)
   // The measurement hook's launch loop, captured once per (kernel, count)
@@ -1192,13 +1063,14 @@ struct GptDecoder::Impl {
     cap = (cap + kChunk - 1) / kChunk * kChunk;
     rows_cap = std::max(std::max(prefix_rows, rows_cap), 16);
     pred_cap = std::max(std::max(steps, pred_cap), 64);
+    chunk_cap = std::min(rows_cap, kPrefillRows);
     const size_t f = sizeof(float);
     size_t bytes = align256(sizeof(GptState)) + align256((size_t)pred_cap * 4) +
                    align256(((size_t)pred_cap + 1) * 4) + 3 * align256(kW * f) + align256(kMLP * f) +
                    align256(kVocab * f) + 2 * align256(kW * f) + align256((size_t)head_blocks() * f) +
                    align256((size_t)head_blocks() * 4) +
-                   3 * align256((size_t)kPrefillRows * kW * f) + align256((size_t)kPrefillRows * kMLP * f) +
-                   align256((size_t)kPrefillRows * kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
+                   3 * align256((size_t)chunk_cap * kW * f) + align256((size_t)chunk_cap * kMLP * f) +
+                   align256((size_t)kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
                    align256((size_t)GptDecoder::kMaxHistory * 4);
     ws.reserve(bytes);
@@ -1214,14 +1086,14 @@ struct GptDecoder::Impl {
     fn = static_cast<float*>(ws.take(kW * f));
     blk_val = static_cast<float*>(ws.take((size_t)head_blocks() * f));
     blk_idx = static_cast<int*>(ws.take((size_t)head_blocks() * 4));
-    xr = static_cast<float*>(ws.take((size_t)kPrefillRows * kW * f));
-    qr = static_cast<float*>(ws.take((size_t)kPrefillRows * kW * f));
-    attr = static_cast<float*>(ws.take((size_t)kPrefillRows * kW * f));
-    fcr = static_cast<float*>(ws.take((size_t)kPrefillRows * kMLP * f));
+    xr = static_cast<float*>(ws.take((size_t)chunk_cap * kW * f));
+    qr = static_cast<float*>(ws.take((size_t)chunk_cap * kW * f));
+    a16 = static_cast<half_t*>(ws.take((size_t)chunk_cap * kW * 2 * sizeof(half_t)));
+    fc16 = static_cast<half_t*>(ws.take((size_t)chunk_cap * kMLP * 2 * sizeof(half_t)));
     proc = static_cast<float*>(ws.take(kVocab * f));
     hist = static_cast<uint32_t*>(ws.take((size_t)GptDecoder::kMaxHistory * 4));
     nsplit_max = cap / kChunk;
-    part = static_cast<float*>(ws.take((size_t)kPrefillRows * kHeads * nsplit_max * kPartF * f));
+    part = static_cast<float*>(ws.take((size_t)kHeads * nsplit_max * kPartF * f));
     kc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
     vc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
     rows = static_cast<float*>(ws.take((size_t)rows_cap * kW * f));
@@ -1246,7 +1118,7 @@ struct GptDecoder::Impl {
       a.w = w.attn_w; a.bias = w.attn_b; a.N = kQKV; a.x = x; a.g1 = w.ln1_w; a.b1 = w.ln1_b;
       a.q = q; a.kc = K; a.vc = V;
       launch_qkv(a, s);
-      launch_attention(q, K, V, att, 1);
+      launch_attention(q, K, V, att);
       a = base_args();
       a.w = w.proj_w; a.bias = w.proj_b; a.N = kW; a.x = att; a.y = x;
       launch_attn_proj(a, s);
@@ -1257,56 +1129,71 @@ struct GptDecoder::Impl {
       a.w = w.mp_w; a.bias = w.mp_b; a.N = kW; a.x = fc; a.y = x; a.advance = l == L - 1;
       launch_mlp_proj(a, s);
     }
-    if (head) {
-      GemvArgs a = base_args();
-      a.w = head_w; a.bias = head_b; a.N = kVocab; a.x = x; a.g1 = lnf_w; a.b1 = lnf_b; a.g2 = fn_w;
-      a.b2 = fn_b; a.y = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.lnf_out = lnf; a.fn_out = fn;
-      launch_head(a, s);
-      if (sample)
-        hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
-                           hist);
-      else
-        hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, head_blocks(), st, predicted,
-                           inputs, 1);
-    }
+    if (head) enqueue_head(x, sample);
     GPT_OK(hipGetLastError());
   }
 
-  // One prefill chunk: up to kPrefillRows prefix rows through every layer.
-  void enqueue_chunk() {
-    hipLaunchKernelGGL(embed_rows_kernel, dim3(1), dim3(256), 0, s, st, rows, xr);
+  // The head on hidden row xv and the token bookkeeping.
+  void enqueue_head(const float* xv, bool sample) {
+    GemvArgs a = base_args();
+    a.w = head_w; a.bias = head_b; a.N = kVocab; a.x = xv; a.g1 = lnf_w; a.b1 = lnf_b; a.g2 = fn_w;
+    a.b2 = fn_b; a.y = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.lnf_out = lnf; a.fn_out = fn;
+    launch_head(a, s);
+    if (sample)
+      hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
+                         hist);
+    else
+      hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, head_blocks(), st, predicted,
+                         inputs, 1);
+  }
+
+  // Prefix rows r0 .. r0 + M - 1 (cache rows of the same numbers) through
+  // every layer together, each product one matrix-core GEMM.  Every weight is
+  // read once per chunk, so a prefix costs about one pass over the weights
+  // and its arithmetic.  The activations are fp32 between the products and
+  // enter each as a split f16 pair (fp32-level products: the weights are
+  // exact in f16); a value that does not fit one sets st->overflow.
+  void enqueue_rows(int r0, int M) {
+    const size_t lo = (size_t)chunk_cap * kW, fc_lo = (size_t)chunk_cap * kMLP;
+    const float* xin = rows + (size_t)r0 * kW;  // the residual stream: the prefix rows, then xr
+    int* ovf = &st->overflow;
+    GemmArgs g;
+    g.M = M;
+    g.split = 1;
     for (int l = 0; l < L; ++l) {
       const GptLayerDev& w = layer[l];
       float* K = kc + (size_t)l * cap * kW;
       float* V = vc + (size_t)l * cap * kW;
-      GemvArgs a = base_args();
-      a.w = w.attn_w; a.bias = w.attn_b; a.N = kQKV; a.x = xr; a.g1 = w.ln1_w; a.b1 = w.ln1_b;
-      a.q = qr; a.kc = K; a.vc = V;
-      launch_rows<kW, 32, 4, PRO_LN, EPI_QKV>(a, s);
-      launch_attention(qr, K, V, attr, kPrefillRows);
-      a = base_args();
-      a.w = w.proj_w; a.bias = w.proj_b; a.N = kW; a.x = attr; a.y = xr;
-      launch_rows<kW, 32, 4, PRO_PLAIN, EPI_RES>(a, s);
-      a = base_args();
-      a.w = w.fc_w; a.bias = w.fc_b; a.N = kMLP; a.x = xr; a.g1 = w.ln2_w; a.b1 = w.ln2_b; a.y = fcr;
-      launch_rows<kW, 32, 4, PRO_LN, EPI_GELU>(a, s);
-      a = base_args();
-      a.w = w.mp_w; a.bias = w.mp_b; a.N = kW; a.x = fcr; a.y = xr;
-      launch_rows<kMLP, 64, 8, PRO_PLAIN, EPI_RES>(a, s);
+      GPT_OK(launch_gpt_ln_rows(xin, w.ln1_w, w.ln1_b, M, a16, lo, ovf, s));
+      GemmArgs a = g;
+      a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.attn_w; a.ldw = kW; a.N = kQKV; a.bias = w.attn_b;
+      a.C32 = qr; a.ldc32 = kW; a.C32b = K; a.C32c = V; a.Tpad = cap; a.T = r0;
+      GPT_OK(launch_gemm_rows(a, EPI_KVCACHE, s));
+      GPT_OK(launch_gpt_attn_rows(qr, K, V, cap, r0, M, a16, lo, ovf, s));
+      a = g;
+      a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.proj_w; a.ldw = kW; a.N = kW; a.bias = w.proj_b;
+      a.res = xin; a.ldres = kW; a.C32 = xr; a.ldc32 = kW;
+      GPT_OK(launch_gemm_rows(a, EPI_F32, s));
+      xin = xr;
+      GPT_OK(launch_gpt_ln_rows(xr, w.ln2_w, w.ln2_b, M, a16, lo, ovf, s));
+      a = g;
+      a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.fc_w; a.ldw = kW; a.N = kMLP; a.bias = w.fc_b;
+      a.C16 = fc16; a.ldc16 = kMLP; a.c16_lo = fc_lo; a.overflow = ovf;
+      GPT_OK(launch_gemm_rows(a, EPI_GELU16, s));
+      a = g;
+      a.A = fc16; a.lda = kMLP; a.a_lo = fc_lo; a.K = kMLP; a.W = w.mp_w; a.ldw = kMLP; a.N = kW; a.bias = w.mp_b;
+      a.res = xr; a.ldres = kW; a.C32 = xr; a.ldc32 = kW;
+      GPT_OK(launch_gemm_rows(a, EPI_F32, s));
     }
-    hipLaunchKernelGGL(advance_rows_kernel, dim3(1), dim3(1), 0, s, st);
-    GPT_OK(hipGetLastError());
   }
 
-  // 0 row, 1 row + head, 2 token + head, 3 prefill chunk, 4 = 2 x kStepsPerCheck,
-  // 5 token + head + sampler, 6 = 5 x kStepsPerCheck
+  // 0 row, 1 row + head, 2 token + head, 3 = 2 x kStepsPerCheck,
+  // 4 token + head + sampler, 5 = 4 x kStepsPerCheck
   void run_step(int which) {
     auto enqueue = [&] {
-      if (which == 3) {
-        enqueue_chunk();
-      } else if (which == 4 || which == 6) {
-        for (int i = 0; i < kStepsPerCheck; ++i) enqueue_step(1, true, which == 6);
-      } else if (which == 5) {
+      if (which == 3 || which == 5) {
+        for (int i = 0; i < kStepsPerCheck; ++i) enqueue_step(1, true, which == 5);
+      } else if (which == 4) {
         enqueue_step(1, true, true);
       } else {
         enqueue_step(which == 2 ? 1 : 0, which != 0);
@@ -1336,19 +1223,30 @@ struct GptDecoder::Impl {
     GPT_OK(hipGraphLaunch(graph[which], s));
   }
 
-  // Prefix rows into the caches: chunks of kPrefillRows rows (env
-  // MIT2CFM_GPT_ROW_PREFILL=1: one row at a time, through the decode
-  // step's kernels -- the same values, for checking).
-  void prefill(int n) {
-    const char* e = std::getenv("MIT2CFM_GPT_ROW_PREFILL");
-    if (e && std::atoi(e) != 0) {
+  // Prefix rows into the caches, in chunks of up to kPrefillRows rows, or one
+  // at a time through the decode step's kernels (`by_rows`: all fp32, whatever
+  // the values' range).  Returns the last row's hidden state (by_rows: NULL).
+  const float* prefill(int n, bool by_rows) {
+    if (by_rows) {
       for (int i = 0; i < n; ++i) run_step(0);
-    } else {
-      for (int i = 0; i < n; i += kPrefillRows) run_step(3);
+      return nullptr;
     }
+    const float* last = nullptr;
+    for (int i = 0; i < n; i += chunk_cap) {
+      const int M = std::min(chunk_cap, n - i);
+      enqueue_rows(i, M);
+      last = xr + (size_t)(M - 1) * kW;
+    }
+    return last;
+  }
+  // env MIT2CFM_GPT_ROW_PREFILL=1: prefill one row at a time (for checking).
+  static bool row_prefill() {
+    const char* e = std::getenv("MIT2CFM_GPT_ROW_PREFILL");
+    return e && std::atoi(e) != 0;
   }
 
-  void reset_state(int prefix_rows, int pend, bool hf, int steps, const GptDecoder::Sampling* smp = nullptr) {
+  // kv: rows the caches hold once the prefill has run (0: rows join one by one)
+  void reset_state(int prefix_rows, int kv, bool hf, const GptDecoder::Sampling* smp = nullptr) {
     GptState h{};
     h.temperature = 1.0f;
     h.top_p = 1.0f;
@@ -1362,7 +1260,7 @@ struct GptDecoder::Impl {
       h.n_hist = (int32_t)smp->n_history;
       h.hist_given = smp->history != nullptr ? 1 : 0;
     }
-    h.kv = 0;
+    h.kv = kv;
     h.step = 0;
     h.n_pred = 0;
     h.n_in = 1;
@@ -1374,8 +1272,6 @@ struct GptDecoder::Impl {
     h.max_pred = pred_cap;
     h.cap = cap;
     h.rows = std::max(prefix_rows, 1);
-    h.pend = pend;
-    (void)steps;
     *host_state = h;
     const uint32_t start = (uint32_t)kStart;
     GPT_OK(hipMemcpyAsync(st, host_state, sizeof(GptState), hipMemcpyHostToDevice, s));
@@ -1527,28 +1423,34 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
                                   std::to_string(kPos) + "-row mel position table");
   }
   d.ensure(prefix_tokens + steps + 1, prefix_tokens + 1, steps);
-  d.reset_state(prefix_tokens, prefix_tokens, hf, steps, sampling);
   if (prefix_tokens > 0)
     GPT_OK(hipMemcpyAsync(d.rows, prefix, (size_t)prefix_tokens * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
-  GPT_OK(hipEventRecord(d.ev[0], d.s));
-  d.prefill(prefix_tokens);
-  GPT_OK(hipEventRecord(d.ev[1], d.s));
-  int done = 0;
-  while (done < steps) {
-    const int n = std::min(kStepsPerCheck, steps - done);
-    if (n == kStepsPerCheck) {
-      d.run_step(sampling ? 6 : 4);  // one graph of kStepsPerCheck steps
-    } else {
-      for (int i = 0; i < n; ++i) d.run_step(sampling ? 5 : 2);
+  auto decode = [&](bool by_rows) {
+    d.reset_state(prefix_tokens, by_rows ? 0 : prefix_tokens, hf, sampling);
+    GPT_OK(hipEventRecord(d.ev[0], d.s));
+    d.prefill(prefix_tokens, by_rows);
+    GPT_OK(hipEventRecord(d.ev[1], d.s));
+    int done = 0;
+    while (done < steps) {
+      const int n = std::min(kStepsPerCheck, steps - done);
+      if (n == kStepsPerCheck) {
+        d.run_step(sampling ? 5 : 3);  // one graph of kStepsPerCheck steps
+      } else {
+        for (int i = 0; i < n; ++i) d.run_step(sampling ? 4 : 2);
+      }
+      done += n;
+      GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
+      GPT_OK(hipStreamSynchronize(d.s));
+      if (d.host_state->stopped || d.host_state->overflow) break;
     }
-    done += n;
+    GPT_OK(hipEventRecord(d.ev[2], d.s));
     GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
     GPT_OK(hipStreamSynchronize(d.s));
-    if (d.host_state->stopped) break;
-  }
-  GPT_OK(hipEventRecord(d.ev[2], d.s));
-  GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
-  GPT_OK(hipStreamSynchronize(d.s));
+    return d.host_state->overflow == 0;
+  };
+  // A prefix whose activations leave f16's range is decoded again from rows
+  // prefilled in fp32.
+  if (d.row_prefill() || !decode(false)) decode(true);
   const GptState h = *d.host_state;
   out.first_stop_step = h.stop_step;
   out.predicted.assign((size_t)h.n_pred, 0);
@@ -1574,12 +1476,21 @@ uint32_t GptDecoder::cached_decode(const float* rows, int prefix_tokens, float* 
   if (prefix_tokens < 0) throw std::invalid_argument("gpt: prefix_tokens must be >= 0");
   if (!rows) throw std::invalid_argument("gpt: rows must not be NULL");
   d.ensure(prefix_tokens + 1, prefix_tokens + 1, 1);
-  d.reset_state(prefix_tokens + 1, prefix_tokens, false, 1);
   GPT_OK(hipMemcpyAsync(d.rows, rows, ((size_t)prefix_tokens + 1) * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
-  d.prefill(prefix_tokens);
-  d.run_step(1);
-  GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
-  GPT_OK(hipStreamSynchronize(d.s));
+  auto decode = [&](bool by_rows) {
+    d.reset_state(prefix_tokens + 1, 0, false);
+    if (by_rows) {
+      d.prefill(prefix_tokens, true);
+      d.run_step(1);
+    } else {  // the last row is known too: it goes through the layers with the others
+      d.enqueue_head(d.prefill(prefix_tokens + 1, false), false);
+      GPT_OK(hipGetLastError());
+    }
+    GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
+    GPT_OK(hipStreamSynchronize(d.s));
+    return d.host_state->overflow == 0;
+  };
+  if (d.row_prefill() || !decode(false)) decode(true);
   if (ln_f) GPT_OK(hipMemcpy(ln_f, d.lnf, kW * sizeof(float), hipMemcpyDeviceToHost));
   if (final_norm) GPT_OK(hipMemcpy(final_norm, d.fn, kW * sizeof(float), hipMemcpyDeviceToHost));
   if (logits) GPT_OK(hipMemcpy(logits, d.logits, kVocab * sizeof(float), hipMemcpyDeviceToHost));
@@ -1611,7 +1522,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
   }
   // A state with kKeys - 1 cached rows; the caches hold whatever they hold
   // (timing only).
-  d.reset_state(1, 0, false, 1);
+  d.reset_state(1, 0, false);
   d.host_state->kv = kKeys - 1;
   GPT_OK(hipMemcpyAsync(d.st, d.host_state, sizeof(GptState), hipMemcpyHostToDevice, d.s));
   GPT_OK(hipMemsetAsync(d.x, 0, kW * sizeof(float), d.s));
@@ -1665,7 +1576,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
         break;
       default:
         d.launch_attention(d.q, d.kc + (size_t)(i % d.L) * d.cap * kW, d.vc + (size_t)(i % d.L) * d.cap * kW,
-                           d.att, 1, 0);
+                           d.att, 0);
         break;
     }
   }

@@ -1,0 +1,24 @@
+// gpt_prefill.h -- row kernels of the GPT decoder's prefill (gpt_prefill.hip):
+// the prefix rows go through each layer together, as split f16 pairs on the
+// matrix cores (launch_gemm_rows) between these LayerNorm and attention
+// kernels.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "device_common.h"
+
+namespace mit2hip {
+
+// y = LayerNorm(x) of M rows of kGptW floats, written as a split f16 pair
+// (y, its lo half at y + y_lo).  Sets *overflow when a value does not fit.
+hipError_t launch_gpt_ln_rows(const float* x, const float* g, const float* b, int M, half_t* y, size_t y_lo,
+                              int* overflow, hipStream_t s);
+
+// Causal attention of M query rows q [M][kGptW] at cache rows kv0 .. kv0 + M - 1
+// over the head-major caches [heads][cap][64], which already hold those rows:
+// row m sees keys 0 .. kv0 + m.  The output is a split f16 pair as above.
+hipError_t launch_gpt_attn_rows(const float* q, const float* kc, const float* vc, int cap, int kv0, int M,
+                                half_t* y, size_t y_lo, int* overflow, hipStream_t s);
+
+}  // namespace mit2hip

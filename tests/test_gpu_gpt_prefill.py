@@ -1,0 +1,103 @@
+"""GPU checks of the GPT decoder's prefill, which pushes the prefix through each
+layer as matrix-core products of split f16 pairs (launch_gemm_rows) with its own
+LayerNorm and attention kernels.
+
+The reference is the same call with MIT2CFM_GPT_ROW_PREFILL=1: one row at a time
+through the decode step's fp32 kernels, which test_gpu_gpt.py holds to the
+oracle.  Both forms sum in fp32 (a split pair holds a value to 2^-22, and the
+weights are exact in f16), so they differ by the order of fp32 sums: logits of
+magnitude about 1 over sums of 1,280 and 5,120 terms, a few 1e-6 measured; the
+bar is test_gpu_gpt.py's 1e-5 for the same comparison.
+
+Row counts (the prefix and the row decoded with it) sit at the edges of the
+16-query attention blocks, the 32- and 64-row tiles and each rule of the tile
+choice, and past the 1,024-row chunk, so that a second chunk attends to the
+first one's keys.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+W = 1280
+
+
+@pytest.fixture(scope="module")
+def gpt2_t(mit2):
+    return mit2.synthetic_gpt_tensors(layers=2)
+
+
+@pytest.fixture(scope="module")
+def ctx2(mit2, tensors, gpt2_t):
+    c = mit2.Context({**tensors, **gpt2_t}, device=0)
+    yield c
+    c.close()
+
+
+def _rows(n, seed):
+    return (np.random.default_rng(seed).standard_normal((n, W)) * 0.05).astype(np.float32)
+
+
+def _both(ctx, rows, monkeypatch):
+    monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
+    got = ctx.gpt_cached_decode(rows, len(rows) - 1)
+    monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
+    ref = ctx.gpt_cached_decode(rows, len(rows) - 1)
+    return got, ref
+
+
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 33, 64, 65, 129, 193, 321, 450, 641, 1024, 1025, 1100])
+def test_prefill_equals_row_prefill(ctx2, monkeypatch, M):
+    rows = _rows(M, M)
+    print(f"prefill M={M}", flush=True)
+    got, ref = _both(ctx2, rows, monkeypatch)
+    errs = [float(np.abs(a - b).max()) for a, b in zip(got[:3], ref[:3])]
+    print(f"  ln_f {errs[0]:.2e} final_norm {errs[1]:.2e} logits {errs[2]:.2e}", flush=True)
+    assert max(errs) <= 1e-5 and got[3] == ref[3]
+
+
+def test_prefill_caches_serve_the_decode(ctx2, monkeypatch):
+    """Tokens decoded after the prefill read the caches it wrote."""
+    prefix = _rows(97, 5)
+    monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
+    got = ctx2.gpt_kv_greedy(prefix, 20)
+    monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
+    ref = ctx2.gpt_kv_greedy(prefix, 20)
+    assert got["predicted"].tolist() == ref["predicted"].tolist()
+    assert np.abs(got["last_logits"] - ref["last_logits"]).max() <= 1e-5
+
+
+@pytest.mark.parametrize("where", ["gelu", "layernorm", "value"])
+def test_values_past_f16_take_the_row_prefill(mit2, tensors, gpt2_t, monkeypatch, where):
+    """A value that does not fit f16 (a c_fc output of 1e5; a LayerNorm output
+    of 1e5; attention outputs of 1e5) is seen, and the call runs again through
+    the fp32 row prefill: the same bits as asking for it."""
+    t = dict(gpt2_t)
+    if where == "gelu":
+        b = np.array(t["gpt.gpt.h.1.mlp.c_fc.bias"], np.float32)
+        b[7] = 1e5
+        t["gpt.gpt.h.1.mlp.c_fc.bias"] = b
+    elif where == "layernorm":
+        b = np.array(t["gpt.gpt.h.0.ln_2.bias"], np.float32)
+        b[1279] = -1e5
+        t["gpt.gpt.h.0.ln_2.bias"] = b
+    else:
+        b = np.array(t["gpt.gpt.h.0.attn.c_attn.bias"], np.float32)
+        b[2 * W + 70] = 1e5
+        t["gpt.gpt.h.0.attn.c_attn.bias"] = b
+    c = mit2.Context({**tensors, **t}, device=0)
+    try:
+        got, ref = _both(c, _rows(21, 9), monkeypatch)
+        for a, b in zip(got[:3], ref[:3]):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
+        assert got[3] == ref[3]
+        monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
+        g = c.gpt_kv_greedy(_rows(21, 9), 12)
+        monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
+        r = c.gpt_kv_greedy(_rows(21, 9), 12)
+        assert g["predicted"].tolist() == r["predicted"].tolist()
+        assert np.array_equal(g["last_logits"], r["last_logits"])
+    finally:
+        c.close()
