@@ -25,7 +25,12 @@
 // (27 passes over the weights) and takes 2.17 ms so; 0.2 ms is what reading the
 // weights once costs, the rest the latency of 24 x 7 dependent launches.
 //
-// Every matrix-vector product is HBM-bound: each weight is read once per
+// A step normally runs as one resident kernel (gpt_token.hip); the kernels
+// below are its plain form, fp32 throughout, one launch a product: for values
+// past f16's range, for a GPU that cannot hold all of that kernel's workgroups
+// at once, and for rows prefilled one by one.
+//
+// Every matrix-vector product reads its weights from HBM: each once per
 // step (f16, 0.98 GB for 24 layers) and used for one multiply-add.  The GEMV
 // kernel loads the input vector, then streams whole rows into registers
 // (16-byte loads, a group of 32 or 64 lanes per row), computes the LayerNorm
@@ -37,18 +42,22 @@
 #include "gpt.h"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <type_traits>
 
 #include "device_common.h"
 #include "engine.h"
-#include "gemm.h"
 #include "gpt_prefill.h"
+#include "gpt_state.h"
+#include "gpt_token.h"
 #include "image_io.h"
 
 namespace mit2hip {
@@ -63,8 +72,6 @@ namespace mit2hip {
 
 namespace {
 
-constexpr int kW = kGptW, kQKV = 3840, kMLP = 5120, kHeads = 20, kHD = 64;
-constexpr int kVocab = GptDecoder::kVocab, kPos = GptDecoder::kPositions;
 constexpr int kStart = (int)GptDecoder::kStartToken, kStop = (int)GptDecoder::kStopToken;
 #ifndef GPT_ATTN_KEYS
 #define GPT_ATTN_KEYS 256
@@ -73,33 +80,6 @@ constexpr int kChunk = GPT_ATTN_KEYS;  // keys per attention split
 static_assert(kChunk % 64 == 0 && kChunk <= 512, "a split is whole passes of 64 keys, one score per thread");
 constexpr int kStepsPerCheck = 8;  // decode steps replayed between stop-flag reads
 constexpr int kPrefillRows = 1024;  // most prefix rows per prefill chunk (36 KB of workspace a row)
-
-// Device-side decode state.
-struct GptState {
-  int32_t kv;         // rows in the key/value caches
-  int32_t step;       // decode steps taken
-  int32_t n_pred;     // predicted tokens written
-  int32_t n_in;       // input tokens written (the start token included)
-  int32_t stopped;    // 1 once the stop token was predicted
-  int32_t stop_step;  // step of the first stop token, else -1
-  int32_t cur_token;  // the last input token
-  int32_t hf;         // position rule: step s > 0 uses position s + 1
-  int32_t argmax;     // argmax of the last head launch
-  int32_t max_pred;   // capacity of the predicted array (inputs: + 1)
-  int32_t cap;        // rows of each key/value cache
-  int32_t rows;       // rows of the prefix buffer
-  int32_t overflow;   // 1: a prefill value did not fit a split f16 pair
-  int32_t top_k;      // sampling (sample_kernel): top-k (0: off)
-  float temperature;  //   temperature, top-p, repetition penalty
-  float top_p;
-  float penalty;
-  int32_t n_hist;     //   repetition-history prefix tokens
-  uint64_t rng;       //   splitmix64 state, advanced once per sampled step
-  int32_t hist_given; //   1: the history starts with the caller's prefix (even an
-                      //   empty one), 0: with the start token
-  int32_t pad[11];
-};
-static_assert(sizeof(GptState) == 128, "GptState layout");
 
 enum { PRO_PLAIN = 0, PRO_LN = 1, PRO_LN2 = 2 };
 enum { EPI_GELU = 0, EPI_RES = 1, EPI_QKV = 2, EPI_LOGITS = 3 };
@@ -940,6 +920,35 @@ void launch_fc(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_FC_SHAPE,
 void launch_mlp_proj(const GemvArgs& a, hipStream_t s) { launch_gemv<kMLP, GPT_MP_SHAPE, PRO_PLAIN, EPI_RES>(a, s); }
 void launch_head(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_HEAD_SHAPE, PRO_LN2, EPI_LOGITS>(a, s); }
 
+// Resident kernels of one device take turns: two at once could each hold CUs
+// that the other waits for.  While a turn lasts, its stream's work is enqueued
+// behind the last turn's; the device event is shared by all contexts.
+class ResidentTurn {
+ public:
+  explicit ResidentTurn(hipStream_t s) : s_(s) {
+    int dev = 0;
+    GPT_OK(hipGetDevice(&dev));
+    static Gate gates[64];
+    gate_ = &gates[dev & 63];
+    lock_ = std::unique_lock<std::mutex>(gate_->m);
+    if (!gate_->ev) {
+      GPT_OK(hipEventCreateWithFlags(&gate_->ev, hipEventDisableTiming));
+    } else {
+      GPT_OK(hipStreamWaitEvent(s_, gate_->ev, 0));
+    }
+  }
+  ~ResidentTurn() { (void)hipEventRecord(gate_->ev, s_); }
+
+ private:
+  struct Gate {
+    std::mutex m;
+    hipEvent_t ev = nullptr;  // the last turn's end (kept for the process)
+  };
+  hipStream_t s_;
+  Gate* gate_;
+  std::unique_lock<std::mutex> lock_;
+};
+
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 }  // namespace
@@ -971,6 +980,8 @@ struct GptDecoder::Impl {
   half_t *a16, *fc16;           //   the products' split operands [2][rows][1280] and [2][rows][5120]
   float* proc = nullptr;        // the sampler's processed logits [8194]
   uint32_t* hist = nullptr;     // the repetition-history prefix [kMaxHistory]
+  TokenMail* mail = nullptr;    // the resident step kernel's words
+  uint32_t epoch = 1;           // first tag epoch no launch has used
   float* part = nullptr;        // attention splits: [20 heads][nsplit_max][66]
   int nsplit_max = 0;
 
@@ -984,9 +995,14 @@ struct GptDecoder::Impl {
   int* blk_idx;
   GptState* host_state = nullptr;  // pinned
   // row, row + head, token + head, kStepsPerCheck token steps, then the
-  // sampled forms of the last two token graphs
-  hipGraphExec_t graph[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  // sampled forms of the last two; the same tokens by the resident kernel
+  hipGraphExec_t graph[10] = {};
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+  // The resident step kernel decodes tokens (else the separate launches do):
+  // all its workgroups fit the device, and no wait of it has run out.
+  bool resident = false;
+  uint32_t spin_limit = 1u << 20;  // env MIT2CFM_GPT_SPIN_LIMIT (for checking: 1 gives up at once)
+  size_t layer_stride = 0;  // bytes from a layer's arrays to the next's
   bool use_graph = true;  // env MIT2CFM_GRAPH=0: launch every kernel directly (for profilers)
   // The measurement hook's launch loop, captured once per (kernel, count)
   // and replayed, so that back-to-back launches are timed without the host's
@@ -1028,6 +1044,37 @@ struct GptDecoder::Impl {
     if (const char* g = std::getenv("MIT2CFM_GRAPH")) use_graph = std::atoi(g) != 0;
     GPT_OK(hipHostMalloc(reinterpret_cast<void**>(&host_state), sizeof(GptState), hipHostMallocDefault));
     for (auto& e : ev) GPT_OK(hipEventCreate(&e));
+    resident = layers_uniform() && gpt_token_fits(current_device());
+    if (const char* g = std::getenv("MIT2CFM_GPT_SPIN_LIMIT")) spin_limit = (uint32_t)std::max(1, std::atoi(g));
+    if (const char* g = std::getenv("MIT2CFM_GPT_RESIDENT")) resident = resident && std::atoi(g) != 0;
+  }
+
+  static int current_device() {
+    int dev = 0;
+    GPT_OK(hipGetDevice(&dev));
+    return dev;
+  }
+  // Whether the layers' arrays lie one stride apart, as a fresh upload and an
+  // image of one lay them out; sets layer_stride.
+  bool layers_uniform() {
+    auto ptrs = [](const GptLayerDev& w) {
+      return std::array<const void*, 12>{w.ln1_w, w.ln1_b, w.attn_w, w.attn_b, w.proj_w, w.proj_b,
+                                         w.ln2_w, w.ln2_b, w.fc_w,   w.fc_b,   w.mp_w,   w.mp_b};
+    };
+    const auto p0 = ptrs(layer[0]);
+    layer_stride = 0;
+    for (int l = 1; l < L; ++l) {
+      const auto p = ptrs(layer[l]);
+      for (size_t i = 0; i < p.size(); ++i) {
+        const ptrdiff_t d = static_cast<const char*>(p[i]) - static_cast<const char*>(p0[i]);
+        if (l == 1 && i == 0) {
+          if (d <= 0) return false;
+          layer_stride = (size_t)d;
+        }
+        if (d != (ptrdiff_t)(layer_stride * (size_t)l)) return false;
+      }
+    }
+    return L <= 64;  // a tag's layer bits
   }
 
   half_t* up_f16(const std::vector<float>& v) {
@@ -1072,7 +1119,7 @@ struct GptDecoder::Impl {
                    3 * align256((size_t)chunk_cap * kW * f) + align256((size_t)chunk_cap * kMLP * f) +
                    align256((size_t)kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
-                   align256((size_t)GptDecoder::kMaxHistory * 4);
+                   align256((size_t)GptDecoder::kMaxHistory * 4) + align256(sizeof(TokenMail));
     ws.reserve(bytes);
     st = static_cast<GptState*>(ws.take(sizeof(GptState)));
     predicted = static_cast<uint32_t*>(ws.take((size_t)pred_cap * 4));
@@ -1093,6 +1140,9 @@ struct GptDecoder::Impl {
     proc = static_cast<float*>(ws.take(kVocab * f));
     hist = static_cast<uint32_t*>(ws.take((size_t)GptDecoder::kMaxHistory * 4));
     nsplit_max = cap / kChunk;
+    mail = static_cast<TokenMail*>(ws.take(sizeof(TokenMail)));
+    GPT_OK(hipMemsetAsync(mail, 0, sizeof(TokenMail), s));  // no word carries a tag yet
+    epoch = 1;
     part = static_cast<float*>(ws.take((size_t)kHeads * nsplit_max * kPartF * f));
     kc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
     vc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
@@ -1133,18 +1183,40 @@ struct GptDecoder::Impl {
     GPT_OK(hipGetLastError());
   }
 
+  // The same token step as one resident kernel and the token bookkeeping.
+  void enqueue_token(bool sample) {
+    const GptLayerDev& w = layer[0];
+    auto c = [](const void* p) { return static_cast<const char*>(p); };
+    TokenArgs a;
+    a.ln1_w = c(w.ln1_w); a.ln1_b = c(w.ln1_b); a.attn_w = c(w.attn_w); a.attn_b = c(w.attn_b);
+    a.proj_w = c(w.proj_w); a.proj_b = c(w.proj_b); a.ln2_w = c(w.ln2_w); a.ln2_b = c(w.ln2_b);
+    a.fc_w = c(w.fc_w); a.fc_b = c(w.fc_b); a.mp_w = c(w.mp_w); a.mp_b = c(w.mp_b);
+    a.stride = layer_stride; a.L = L;
+    a.lnf_w = lnf_w; a.lnf_b = lnf_b; a.fn_w = fn_w; a.fn_b = fn_b; a.head_b = head_b; a.head_w = head_w;
+    a.mel_emb = mel_emb; a.pos_emb = pos_emb;
+    a.st = st; a.kc = kc; a.vc = vc; a.cap = cap; a.mail = mail;
+    a.logits = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.spin_limit = spin_limit;
+    GPT_OK(launch_gpt_token(a, s));
+    enqueue_pick(sample, kTokWG);
+  }
+
+  // The next token from the logits (nb: workgroups that left a maximum).
+  void enqueue_pick(bool sample, int nb) {
+    if (sample)
+      hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
+                         hist);
+    else
+      hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, nb, st, predicted, inputs, 1);
+    GPT_OK(hipGetLastError());
+  }
+
   // The head on hidden row xv and the token bookkeeping.
   void enqueue_head(const float* xv, bool sample) {
     GemvArgs a = base_args();
     a.w = head_w; a.bias = head_b; a.N = kVocab; a.x = xv; a.g1 = lnf_w; a.b1 = lnf_b; a.g2 = fn_w;
     a.b2 = fn_b; a.y = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.lnf_out = lnf; a.fn_out = fn;
     launch_head(a, s);
-    if (sample)
-      hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
-                         hist);
-    else
-      hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, head_blocks(), st, predicted,
-                         inputs, 1);
+    enqueue_pick(sample, head_blocks());
   }
 
   // Prefix rows r0 .. r0 + M - 1 (cache rows of the same numbers) through
@@ -1188,15 +1260,20 @@ struct GptDecoder::Impl {
   }
 
   // 0 row, 1 row + head, 2 token + head, 3 = 2 x kStepsPerCheck,
-  // 4 token + head + sampler, 5 = 4 x kStepsPerCheck
+  // 4 token + head + sampler, 5 = 4 x kStepsPerCheck; 6 .. 9: 2 .. 5 by the
+  // resident kernel
   void run_step(int which) {
     auto enqueue = [&] {
-      if (which == 3 || which == 5) {
-        for (int i = 0; i < kStepsPerCheck; ++i) enqueue_step(1, true, which == 5);
-      } else if (which == 4) {
-        enqueue_step(1, true, true);
-      } else {
-        enqueue_step(which == 2 ? 1 : 0, which != 0);
+      if (which < 2) {
+        enqueue_step(0, which == 1);
+        return;
+      }
+      const int kind = which < 6 ? which : which - 4;
+      for (int i = 0; i < (kind & 1 ? kStepsPerCheck : 1); ++i) {
+        if (which < 6)
+          enqueue_step(1, true, kind >= 4);
+        else
+          enqueue_token(kind >= 4);
       }
     };
     if (!use_graph) {
@@ -1246,8 +1323,11 @@ struct GptDecoder::Impl {
   }
 
   // kv: rows the caches hold once the prefill has run (0: rows join one by one)
-  void reset_state(int prefix_rows, int kv, bool hf, const GptDecoder::Sampling* smp = nullptr) {
+  // steps: an upper bound of the steps that follow
+  void reset_state(int prefix_rows, int kv, bool hf, int steps, const GptDecoder::Sampling* smp = nullptr) {
     GptState h{};
+    h.epoch = epoch;
+    epoch += (uint32_t)steps;
     h.temperature = 1.0f;
     h.top_p = 1.0f;
     h.penalty = 1.0f;
@@ -1425,32 +1505,46 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   d.ensure(prefix_tokens + steps + 1, prefix_tokens + 1, steps);
   if (prefix_tokens > 0)
     GPT_OK(hipMemcpyAsync(d.rows, prefix, (size_t)prefix_tokens * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
-  auto decode = [&](bool by_rows) {
-    d.reset_state(prefix_tokens, by_rows ? 0 : prefix_tokens, hf, sampling);
+  auto decode = [&](bool plain) {
+    d.reset_state(prefix_tokens, plain ? 0 : prefix_tokens, hf, steps, sampling);
     GPT_OK(hipEventRecord(d.ev[0], d.s));
-    d.prefill(prefix_tokens, by_rows);
+    d.prefill(prefix_tokens, plain);
     GPT_OK(hipEventRecord(d.ev[1], d.s));
     int done = 0;
     while (done < steps) {
       const int n = std::min(kStepsPerCheck, steps - done);
-      if (n == kStepsPerCheck) {
-        d.run_step(sampling ? 5 : 3);  // one graph of kStepsPerCheck steps
-      } else {
-        for (int i = 0; i < n; ++i) d.run_step(sampling ? 4 : 2);
+      const bool resident = d.resident && !plain;
+      const int token = (sampling ? 4 : 2) + (resident ? 4 : 0);
+      {
+        std::unique_ptr<ResidentTurn> turn(resident ? new ResidentTurn(d.s) : nullptr);
+        if (n == kStepsPerCheck) {
+          d.run_step(token + 1);  // one graph of kStepsPerCheck steps
+        } else {
+          for (int i = 0; i < n; ++i) d.run_step(token);
+        }
       }
       done += n;
       GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
       GPT_OK(hipStreamSynchronize(d.s));
-      if (d.host_state->stopped || d.host_state->overflow) break;
+      if (d.host_state->stopped || d.host_state->overflow || d.host_state->aborted) break;
     }
     GPT_OK(hipEventRecord(d.ev[2], d.s));
     GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
     GPT_OK(hipStreamSynchronize(d.s));
-    return d.host_state->overflow == 0;
+    return d.host_state->overflow == 0 && d.host_state->aborted == 0;
   };
-  // A prefix whose activations leave f16's range is decoded again from rows
-  // prefilled in fp32.
-  if (d.row_prefill() || !decode(false)) decode(true);
+  // A call whose activations leave f16's range runs again the plain way, fp32
+  // throughout: rows prefilled one by one, tokens by the separate launches.
+  // One whose resident kernel had to give up (its workgroups could not all
+  // run: another process keeps some of the GPU's CUs) runs again with those
+  // launches, as do all that follow in this context.
+  bool plain = d.row_prefill();
+  while (!decode(plain)) {
+    if (d.host_state->aborted)
+      d.resident = false;
+    else
+      plain = true;
+  }
   const GptState h = *d.host_state;
   out.first_stop_step = h.stop_step;
   out.predicted.assign((size_t)h.n_pred, 0);
@@ -1478,7 +1572,7 @@ uint32_t GptDecoder::cached_decode(const float* rows, int prefix_tokens, float* 
   d.ensure(prefix_tokens + 1, prefix_tokens + 1, 1);
   GPT_OK(hipMemcpyAsync(d.rows, rows, ((size_t)prefix_tokens + 1) * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
   auto decode = [&](bool by_rows) {
-    d.reset_state(prefix_tokens + 1, 0, false);
+    d.reset_state(prefix_tokens + 1, 0, false, 1);
     if (by_rows) {
       d.prefill(prefix_tokens, true);
       d.run_step(1);
@@ -1522,7 +1616,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
   }
   // A state with kKeys - 1 cached rows; the caches hold whatever they hold
   // (timing only).
-  d.reset_state(1, 0, false);
+  d.reset_state(1, 0, false, 1);
   d.host_state->kv = kKeys - 1;
   GPT_OK(hipMemcpyAsync(d.st, d.host_state, sizeof(GptState), hipMemcpyHostToDevice, d.s));
   GPT_OK(hipMemsetAsync(d.x, 0, kW * sizeof(float), d.s));

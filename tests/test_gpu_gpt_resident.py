@@ -1,0 +1,168 @@
+"""GPU checks of the GPT decode step as one resident kernel (gpt_token.hip).
+
+The reference is the same call on a context created with MIT2CFM_GPT_RESIDENT=0,
+whose steps are separate fp32 launches that test_gpu_gpt.py holds to the oracle.
+The resident kernel's products are split f16 pairs on the matrix cores (a pair
+holds a value to 2^-22, the weights are exact in f16) with fp32 sums, so the two
+differ by the order of fp32 sums of up to 5,120 terms: logits of magnitude about
+1 agree to a few 1e-6, and the bar is test_gpu_gpt.py's 1e-5 for such pairs.
+
+A head's keys are split over four workgroups (row r to workgroup r % 4), each of
+which holds 208 of its rows in LDS and reads the rest from memory, so cache
+lengths run over every remainder of 4, from empty, and across 832.
+"""
+from __future__ import annotations
+
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+W = 1280
+SAMPLING = dict(temperature=0.8, top_k=30, top_p=0.8, repetition_penalty=10.0)
+
+
+def _tensors(mit2, tensors, layers):
+    t = {**tensors, **mit2.synthetic_gpt_tensors(layers=layers)}
+    b = np.array(t["gpt.mel_head.bias"], np.float32)
+    b[mit2.GPT_STOP_TOKEN] -= 20.0  # no early stop
+    t["gpt.mel_head.bias"] = b
+    return t
+
+
+def _plain(mit2, t, monkeypatch):
+    monkeypatch.setenv("MIT2CFM_GPT_RESIDENT", "0")
+    c = mit2.Context(t, device=0)
+    monkeypatch.delenv("MIT2CFM_GPT_RESIDENT")
+    return c
+
+
+@pytest.fixture(scope="module")
+def pair2(mit2, tensors):
+    t = _tensors(mit2, tensors, 2)
+    mp = pytest.MonkeyPatch()
+    a, b = mit2.Context(t, device=0), _plain(mit2, t, mp)
+    mp.undo()
+    yield a, b
+    a.close()
+    b.close()
+
+
+def _rows(n, seed):
+    return (np.random.default_rng(seed).standard_normal((n, W)) * 0.05).astype(np.float32)
+
+
+def _same(a, b):
+    assert a["predicted"].tolist() == b["predicted"].tolist()
+    assert a["input_tokens"].tolist() == b["input_tokens"].tolist()
+    err = float(np.abs(a["last_logits"] - b["last_logits"]).max())
+    print(f"  logits max-abs {err:.2e}", flush=True)
+    assert err <= 1e-5
+
+
+@pytest.mark.parametrize("P,steps", [(0, 1), (0, 9), (1, 3), (2, 1), (3, 8), (65, 17), (827, 1), (828, 12), (1100, 3)])
+def test_greedy_equals_separate_launches(pair2, P, steps):
+    print(f"resident greedy P={P} steps={steps}", flush=True)
+    x = _rows(P, P)
+    _same(pair2[0].gpt_kv_greedy(x, steps, True), pair2[1].gpt_kv_greedy(x, steps, True))
+
+
+@pytest.mark.parametrize("layers", [1, 3])
+def test_layer_counts(mit2, tensors, monkeypatch, layers):
+    t = _tensors(mit2, tensors, layers)
+    a, b = mit2.Context(t, device=0), _plain(mit2, t, monkeypatch)
+    try:
+        print(f"resident greedy layers={layers}", flush=True)
+        _same(a.gpt_kv_greedy(_rows(7, 1), 9), b.gpt_kv_greedy(_rows(7, 1), 9))
+    finally:
+        a.close()
+        b.close()
+
+
+def test_sampled_equals_separate_launches(pair2):
+    x = _rows(33, 2)
+    a, b = (c.gpt_kv_sample(x, 20, 11, hf_generate_positions=True, history=[1] * 33 + [8192], **SAMPLING) for c in pair2)
+    _same(a, b)
+
+
+def test_repeats_to_the_bit(pair2):
+    """The order of every sum is fixed, whichever workgroup comes first."""
+    x = _rows(40, 3)
+    a = pair2[0].gpt_kv_greedy(x, 30)
+    for _ in range(5):
+        b = pair2[0].gpt_kv_greedy(x, 30)
+        assert a["predicted"].tolist() == b["predicted"].tolist()
+        assert np.array_equal(a["last_logits"], b["last_logits"])
+
+
+def test_contexts_on_threads_take_turns(mit2, tensors):
+    """Two contexts decode at once from two threads: their resident kernels run
+    one after the other, and each gives what it gives alone."""
+    t = _tensors(mit2, tensors, 2)
+    ctx = [mit2.Context(t, device=0) for _ in range(2)]
+    try:
+        want = [c.gpt_kv_greedy(_rows(20 + i, i), 60) for i, c in enumerate(ctx)]
+        got = [[], []]
+
+        def work(i):
+            for _ in range(4):
+                got[i].append(ctx[i].gpt_kv_greedy(_rows(20 + i, i), 60))
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        for i in range(2):
+            assert len(got[i]) == 4
+            for g in got[i]:
+                assert g["predicted"].tolist() == want[i]["predicted"].tolist()
+                assert np.array_equal(g["last_logits"], want[i]["last_logits"])
+    finally:
+        for c in ctx:
+            c.close()
+
+
+def test_a_wait_that_runs_out_falls_back(mit2, tensors, monkeypatch):
+    """With a limit of one poll the kernel gives up at its first wait and ends;
+    the call decodes with the separate launches: their bits."""
+    t = _tensors(mit2, tensors, 2)
+    b = _plain(mit2, t, monkeypatch)
+    monkeypatch.setenv("MIT2CFM_GPT_SPIN_LIMIT", "1")
+    a = mit2.Context(t, device=0)
+    try:
+        x = _rows(25, 4)
+        ra, rb = a.gpt_kv_greedy(x, 12), b.gpt_kv_greedy(x, 12)
+        assert ra["predicted"].tolist() == rb["predicted"].tolist()
+        assert np.array_equal(ra["last_logits"], rb["last_logits"])
+        ra = a.gpt_kv_sample(x, 12, 5, **SAMPLING)
+        rb = b.gpt_kv_sample(x, 12, 5, **SAMPLING)
+        assert ra["predicted"].tolist() == rb["predicted"].tolist()
+        assert np.array_equal(ra["last_logits"], rb["last_logits"])
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("where", ["gelu", "layernorm"])
+def test_decode_values_past_f16(mit2, tensors, monkeypatch, where):
+    """A decode step whose values do not fit f16 (nothing of the prefix does,
+    as there is none) runs again through the fp32 launches: their bits."""
+    t = _tensors(mit2, tensors, 2)
+    name, at, v = {"gelu": ("gpt.gpt.h.1.mlp.c_fc.bias", 5119, 1e5),
+                   "layernorm": ("gpt.final_norm.bias", 3, -1e5)}[where]
+    bias = np.array(t[name], np.float32)
+    bias[at] = v
+    t[name] = bias
+    a, b = mit2.Context(t, device=0), _plain(mit2, t, monkeypatch)
+    try:
+        for _ in range(2):
+            ra, rb = a.gpt_kv_greedy(_rows(0, 0), 10), b.gpt_kv_greedy(_rows(0, 0), 10)
+            assert ra["predicted"].tolist() == rb["predicted"].tolist()
+            assert np.isfinite(ra["last_logits"]).all()
+            assert np.array_equal(ra["last_logits"], rb["last_logits"])
+    finally:
+        a.close()
+        b.close()
