@@ -64,6 +64,7 @@ enum EpiMode : int {
   EPI_KVCACHE = 10,   // N = 3 x kGptW, v = acc + bias: columns < kGptW -> C32; the next kGptW
                       // -> C32b and the rest -> C32c, the head-major caches
                       // [head][Tpad rows][64], at cache row T + m
+  EPI_ROWS = 11,      // C32 = acc + bias + res
 };
 
 struct GemmArgs {
@@ -83,6 +84,7 @@ struct GemmArgs {
   int n_store = 0;  // if nonzero: only columns < n_store are stored (weights zero-padded to N)
   const half_t* A_zero = nullptr;  // A_CONVP: >= conv_c zero halves, read by the padding taps
   int conv_window = 1;             // A_CONVP with M = T: 0 streams every tap's rows (no A_CONVW)
+  int peers = 1;                   // A_CONVP: products in this one's launch (launch_gemm_group sets it)
   uint32_t conv_magic = 0;         // A_CONVW, set by launch_gemm: ceil(2^32 / conv_c), so that
                                    // k / conv_c = umulhi(k, conv_magic) for k conv_c < 2^32
   // weights
@@ -216,9 +218,22 @@ constexpr int kSsqParts = 16;
 // launch error.  Host-side checks reject shapes the kernels do not cover.
 hipError_t launch_gemm(const GemmArgs& a, AMode amode, EpiMode epi, hipStream_t stream);
 
+// Most products of one launch.
+constexpr int kMaxGroup = 3;
+
+// n <= kMaxGroup independent products of one shape but for K (the same
+// position of a stage's resblocks, A_CONVP) in one launch, longest K first:
+// their tiles fill the chip together.  Where they need different kernels,
+// or do better apart, one launch each (*together, when given, says which).
+// The same bits as launch_gemm gives.
+hipError_t launch_gemm_group(const GemmArgs* a, int n, AMode amode, EpiMode epi, hipStream_t stream,
+                             bool* together = nullptr);
+
 // The GPT prefill's products: A_PLAIN with a split A and an f16-exact W
-// (GemmArgs::split = 1), epilogue EPI_KVCACHE, EPI_GELU16 or EPI_F32 (with a
-// residual).  K a multiple of 256, N of 64.
+// (GemmArgs::split = 1), epilogue EPI_KVCACHE, EPI_GELU16 or EPI_ROWS.  K a
+// multiple of 256, N of 64.  Each K stage is summed by itself before it joins
+// the total (over the whole stack an error against float64 of 3.6e-7, as the
+// vector units gave; 7e-7 as one chain).
 hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream);
 
 }  // namespace mit2hip

@@ -119,8 +119,24 @@ __device__ inline half_t f16_of(float v) {
   return (half_t)v;
 }
 
-template <int BM, int BN, int SK, int NST, int AM, int EPI, int WM, int WN, int KG, int SP, int PIPE>
-__global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(GemmArgs p, TileMap tmap) {
+// The products of one launch: product i's workgroups start at first[i].
+template <int G>
+struct GemmGroup {
+  GemmArgs p[G];
+  TileMap t[G];
+  int first[G];
+};
+
+template <int BM, int BN, int SK, int NST, int AM, int EPI, int WM, int WN, int KG, int SP, int PIPE, int GRP = 1>
+__global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(GemmGroup<GRP> grp) {
+  int gi = 0;
+  if constexpr (GRP > 1) {
+#pragma unroll
+    for (int i = 1; i < GRP; ++i) gi = (int)blockIdx.x >= grp.first[i] ? i : gi;
+  }
+  const GemmArgs& p = grp.p[gi];
+  const TileMap& tmap = grp.t[gi];
+  const int block = GRP > 1 ? (int)blockIdx.x - grp.first[gi] : (int)blockIdx.x;
   // K split.  The product over K is summed in KG parts of equal length, added
   // in part order at the end (the same bits whichever form computes them).
   // PIPE = 0: part g is walked by its own group of WM x WN wavefronts with
@@ -213,7 +229,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
   };
 
   int tile_m, tile_n;
-  if (!tmap.map(blockIdx.x, tile_m, tile_n)) return;
+  if (!tmap.map(block, tile_m, tile_n)) return;
   const int m0 = tile_m * BM;
   const int n0 = tile_n * BN;
 
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
   // the K loop, so their latency hides behind it (PIPE = 1: after the loop,
   // so they do not hold registers beside its larger tiles).
   constexpr bool kPreA =
-      EPI == EPI_F32 || EPI == EPI_RESSKIP || EPI == EPI_FINALSKIP || EPI == EPI_RESAVG;
+      EPI == EPI_F32 || EPI == EPI_RESSKIP || EPI == EPI_FINALSKIP || EPI == EPI_RESAVG || EPI == EPI_ROWS;
   constexpr bool kPreB = EPI == EPI_FINALSKIP;
   // The WaveNet epilogues' row mask (one word per row) and the gate's
   // global conditioning (one float4 pair per column group) as well: fetched
@@ -303,7 +319,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
         const int n = colj(j);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (m < p.M && kg == 0 && (p.n_store == 0 || n < p.n_store)) {
-          if constexpr (EPI == EPI_F32 || EPI == EPI_RESAVG) {
+          if constexpr (EPI == EPI_F32 || EPI == EPI_RESAVG || EPI == EPI_ROWS) {
             if (p.res) v = *reinterpret_cast<const float4*>(p.res + (size_t)m * p.ldres + n);
           }
         }
@@ -588,15 +604,16 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
       for (int j = 0; j < NI; ++j) accx[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
   // The GPT prefill's long sums: each stage's product is summed by itself and
-  // then added to the total, so no value passes through a chain of K / 32
-  // matrix-core additions.
-  constexpr bool kFold = AM == A_PLAIN && SP == 1;
-  floatx4 tot[kFold ? MI : 1][kFold ? NI : 1];
+  // added to a partial sum, and that to the total every eight stages, so no
+  // value passes through a chain of K / 32 matrix-core additions.
+  constexpr bool kFold = EPI == EPI_ROWS || EPI == EPI_GELU16 || EPI == EPI_KVCACHE;
+  static_assert(!kFold || SP == 1, "the GPT prefill's operands");
+  floatx4 tot[kFold ? MI : 1][kFold ? NI : 1], tot8[kFold ? MI : 1][kFold ? NI : 1];
   if constexpr (kFold) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) tot[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NI; ++j) tot[i][j] = tot8[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
   // Fragment reads.  Every fragment row of this lane has the same swizzle
@@ -671,9 +688,18 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-          tot[i][j] += acc[i][j];
+          tot8[i][j] += acc[i][j];
           acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
+      if ((kt & 7) == 7) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) {
+            tot[i][j] += tot8[i][j];
+            tot8[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
     }
   };
 
@@ -867,7 +893,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j];
+      for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j] + tot8[i][j];
   }
   if constexpr (SP > 0) {
 #pragma unroll
@@ -958,7 +984,8 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
                                                       nsa[j].z * nsg[j].z, nsa[j].w * nsg[j].w);
   }
   if constexpr (EPI == EPI_F32 || EPI == EPI_F16 || EPI == EPI_DUAL || EPI == EPI_RESSKIP ||
-                EPI == EPI_FINALSKIP || EPI == EPI_RESAVG || EPI == EPI_GELU16 || EPI == EPI_KVCACHE) {
+                EPI == EPI_FINALSKIP || EPI == EPI_RESAVG || EPI == EPI_GELU16 || EPI == EPI_KVCACHE ||
+                EPI == EPI_ROWS) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       const int m = row_base + 16 * i;
@@ -1028,6 +1055,10 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
         if (!live) continue;
         if constexpr (EPI == EPI_F16) {
           st16s(p.C16 + (size_t)m * p.ldc16 + n, v.x, v.y, v.z, v.w);
+        } else if constexpr (EPI == EPI_ROWS) {
+          const float4 r = pre_a[i][j];
+          *reinterpret_cast<float4*>(p.C32 + (size_t)m * p.ldc32 + n) =
+              make_float4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
         } else if constexpr (EPI == EPI_GELU16) {
           const float4 y = make_float4(gelu_new(v.x), gelu_new(v.y), gelu_new(v.z), gelu_new(v.w));
           // (written so that a NaN counts as not fitting)
@@ -1494,12 +1525,23 @@ static TileMap make_tile_map(const GemmArgs& a, int M, int N, int K, int a_cols,
   }
   const double a_bytes = 2.0 * M * a_cols, w_bytes = 2.0 * N * K;
   const int opts[4][2] = {{8, 1}, {4, 2}, {2, 4}, {1, 8}};
+  auto most = [&](int xm, int xn) { return ((t.nM + xm - 1) / xm) * ((t.nN + xn - 1) / xn); };  // an XCD's tiles
+  // The vocoder's convs (6 or 3 column tiles in their wide stages) split
+  // unevenly into some rectangles, 28 tiles for one XCD and 13 for another:
+  // no matter for a product of one round, but a launch of several, or of three
+  // products, waits for the fullest XCD.  They take a rectangle within an
+  // eighth of the evenest.
+  int even = 1 << 30;
+  if (a.conv_k > 0)
+    for (const auto& o : opts)
+      if (o[0] <= t.nM && o[1] <= t.nN) even = std::min(even, most(o[0], o[1]));
   double best = 1e300;
   t.Xm = 8;
   t.Xn = 1;
   for (const auto& o : opts) {
     const int xm = o[0], xn = o[1];
     if (xm > t.nM || xn > t.nN) continue;
+    if (even < (1 << 30) && most(xm, xn) > even + even / 8) continue;
     const double cost = a_bytes * xn + w_bytes * xm;
     if (cost < best) {
       best = cost;
@@ -1522,17 +1564,42 @@ static TileMap make_tile_map(const GemmArgs& a, int M, int N, int K, int a_cols,
   return t;
 }
 
+// A launch that launch_gemm_group holds back: the kernel for one product and
+// for kMaxGroup of them.
+struct HeldLaunch {
+  GemmArgs a;
+  TileMap t;
+  dim3 block;
+  bool one_round = false;  // a pipelined tiling of at most one workgroup per CU
+  void (*one)(GemmGroup<1>) = nullptr;
+  void (*group)(GemmGroup<kMaxGroup>) = nullptr;
+};
+static thread_local HeldLaunch* t_hold = nullptr;
+
 template <int BM, int BN, int SK, int NST, int AM, int EPI, int WM = 2, int WN = 2, int KG = 1,
           int SP = 0, int PIPE = 0>
 static hipError_t launch_tile(const GemmArgs& a, hipStream_t s) {
   if ((a.K / SK) % KG != 0) return hipErrorInvalidValue;  // both K parts need equal stage counts
   if (PIPE && (a.K / SK / KG) % NST != 0) return hipErrorInvalidValue;  // whole rounds per part
-  const TileMap tm = make_tile_map(
+  GemmGroup<1> g;
+  g.p[0] = a;
+  g.t[0] = make_tile_map(
       a, a.M, a.N, a.K, AM == A_CONV5 || AM == A_CONV3Z || AM == A_CONVP || AM == A_CONVW ? a.conv_c : a.K,
       BM, BN);
-  hipLaunchKernelGGL((gemm_kernel<BM, BN, SK, NST, AM, EPI, WM, WN, KG, SP, PIPE>), dim3(8 * tm.per_xcd),
-                     dim3(64 * WM * WN * (PIPE ? 1 : KG)), 0, s,
-                     a, tm);
+  g.first[0] = 0;
+  const dim3 block(64 * WM * WN * (PIPE ? 1 : KG));
+  auto one = gemm_kernel<BM, BN, SK, NST, AM, EPI, WM, WN, KG, SP, PIPE>;
+  if (t_hold) {
+    t_hold->a = a;
+    t_hold->t = g.t[0];
+    t_hold->block = block;
+    t_hold->one = one;
+    t_hold->one_round = PIPE && g.t[0].nM * g.t[0].nN <= 256;
+    if constexpr ((AM == A_CONVP || AM == A_CONVW) && EPI == EPI_F32)
+      t_hold->group = gemm_kernel<BM, BN, SK, NST, AM, EPI, WM, WN, KG, SP, PIPE, kMaxGroup>;
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(one, dim3(8 * g.t[0].per_xcd), block, 0, s, g);
   return hipGetLastError();
 }
 
@@ -1688,6 +1755,25 @@ static bool launch_conv_window(const GemmArgs& a0, hipStream_t s, hipError_t& e)
   return false;
 }
 
+// The wide convs of a short call (a few hundred rows): smaller tiles than
+// 64 x 128, so that more CUs take part; the time is the latency of the K stages.
+template <int EPI, int SP>
+static bool launch_conv_rows(const GemmArgs& a, hipStream_t s, hipError_t& e) {
+  if (a.N % 128 != 0 || a.row_nb != 0) return false;
+  const long t = tile_count(a, 64, 128);
+  constexpr int kDeep = SP == 0 ? 6 : SP == 1 ? 5 : 3;  // stages that leave room for two workgroups a CU
+  if (t <= 32) {
+    e = launch_tile<32, 64, 64, kDeep, A_CONVP, EPI, 2, 2, 1, SP>(a, s);
+  } else if (t <= 64) {
+    e = launch_tile<32, 64, 64, 3, A_CONVP, EPI, 2, 2, 1, SP>(a, s);
+  } else if (t <= 100 && SP < 2) {
+    e = launch_tile<64, 64, 64, SP == 0 ? 4 : 3, A_CONVP, EPI, 4, 2, 1, SP>(a, s);
+  } else {
+    return false;
+  }
+  return true;
+}
+
 template <int AM, int EPI, int SP>
 static hipError_t launch_split(const GemmArgs& a, hipStream_t s) {
   if constexpr (AM == A_CONVP) {
@@ -1711,6 +1797,10 @@ static hipError_t launch_split(const GemmArgs& a, hipStream_t s) {
         return launch_tile<64, 96, 64, 3, AM, EPI, 4, 1, 1, SP>(a, s);
       }
     }
+    if constexpr (EPI == EPI_F32) {
+      hipError_t e;
+      if (launch_conv_rows<EPI, SP>(a, s, e)) return e;
+    }
     if (a.N % 128 == 0) return launch_tile<64, 128, 64, 3, AM, EPI, 2, 4, 1, SP>(a, s);
     if (a.N % 64 == 0) return launch_tile<64, 64, 64, 3, AM, EPI, 2, 2, 1, SP>(a, s);
     if (a.N % 32 == 0) return launch_tile<64, 32, 64, 3, AM, EPI, 4, 1, 1, SP>(a, s);
@@ -1732,6 +1822,10 @@ static hipError_t launch_am_epi(const GemmArgs& a, hipStream_t s) {
     if constexpr (EPI == EPI_F32 || EPI == EPI_RESAVG) {
       hipError_t e;
       if (a.conv_window && a.M == a.T && a.row_nb == 0 && launch_conv_window<EPI, 0>(a, s, e)) return e;
+    }
+    if constexpr (EPI == EPI_F32) {
+      hipError_t e;
+      if (launch_conv_rows<EPI, 0>(a, s, e)) return e;
     }
     if (a.N % 128 == 0) return launch_tile<64, 128, 64, 3, AM, EPI, 2, 4>(a, s);
     if (a.N % 64 == 0) return launch_tile<64, 64, 64, 3, AM, EPI, 2, 2>(a, s);
@@ -1894,6 +1988,51 @@ hipError_t launch_gemm(const GemmArgs& a, AMode amode, EpiMode epi, hipStream_t 
   return hipErrorInvalidValue;  // combination not built
 }
 
+hipError_t launch_gemm_group(const GemmArgs* a, int n, AMode amode, EpiMode epi, hipStream_t stream, bool* together) {
+  if (n < 1 || n > kMaxGroup || amode != A_CONVP) return hipErrorInvalidValue;
+  HeldLaunch h[kMaxGroup];
+  bool same = n == kMaxGroup;
+  for (int i = 0; i < n; ++i) {
+    GemmArgs g = a[i];
+    g.peers = n;
+    t_hold = &h[i];
+    const hipError_t e = launch_gemm(g, amode, epi, stream);
+    t_hold = nullptr;
+    if (e != hipSuccess) return e;
+    same = same && h[i].group && h[i].group == h[0].group && a[i].M == a[0].M && a[i].N == a[0].N;
+    // (the pipelined kernel fills a CU's LDS, so tiles of one product take no
+    // room beside another's: three products of one round each ran 0.05 to 0.1
+    // ms a launch slower together, at 2,800 to 4,800 rows of 768 channels)
+    same = same && !h[i].one_round;
+  }
+  if (together) *together = same;
+  if (same) {
+    int order[kMaxGroup];
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::sort(order, order + n, [&](int x, int y) { return a[x].K > a[y].K; });
+    GemmGroup<kMaxGroup> g;
+    int blocks = 0;  // (a multiple of 8 before each product: its tiles keep their XCDs)
+    for (int i = 0; i < n; ++i) {
+      g.p[i] = h[order[i]].a;
+      g.t[i] = h[order[i]].t;
+      g.first[i] = blocks;
+      blocks += 8 * g.t[i].per_xcd;
+    }
+    hipLaunchKernelGGL(h[0].group, dim3(blocks), h[0].block, 0, stream, g);
+    return hipGetLastError();
+  }
+  for (int i = 0; i < n; ++i) {
+    GemmGroup<1> g;
+    g.p[0] = h[i].a;
+    g.t[0] = h[i].t;
+    g.first[0] = 0;
+    hipLaunchKernelGGL(h[i].one, dim3(8 * g.t[0].per_xcd), h[i].block, 0, stream, g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 // GPT prefill products (split A, W exact in f16; layer shapes N x K 3840 x
 // 1280, 1280 x 1280, 5120 x 1280 and 1280 x 5120).  A few hundred rows make a
 // few hundred tiles at most, whose time is the latency of their K stages (the
@@ -1917,7 +2056,7 @@ static hipError_t launch_rows_epi(const GemmArgs& a, hipStream_t s) {
   if (t64 > 256) return launch_tile<64, 64, 64, 3, A_PLAIN, EPI, 4, 2, 1, 1>(a, s);
   if (t64 > 128) return launch_tile<64, 64, 64, 4, A_PLAIN, EPI, 4, 2, 1, 1>(a, s);
   if (tile_count(a, 32, 32) <= 160) return launch_tile<32, 32, 64, 3, A_PLAIN, EPI, 2, 1, 4, 1>(a, s);
-  if (EPI == EPI_F32 && a.K >= 2560) return launch_tile<64, 32, 64, 3, A_PLAIN, EPI, 4, 1, 2, 1>(a, s);
+  if (EPI == EPI_ROWS && a.K >= 2560) return launch_tile<64, 32, 64, 3, A_PLAIN, EPI, 4, 1, 2, 1>(a, s);
   return launch_tile<32, 64, 64, 5, A_PLAIN, EPI, 2, 2, 1, 1>(a, s);
 }
 
@@ -1928,7 +2067,7 @@ hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream) 
   if (epi == EPI_KVCACHE && a.N == 3 * kGptW && a.C32 && a.C32b && a.C32c && a.T >= 0 && a.T + a.M <= a.Tpad)
     return launch_rows_epi<EPI_KVCACHE>(a, stream);
   if (epi == EPI_GELU16 && a.C16 && a.c16_lo && a.overflow) return launch_rows_epi<EPI_GELU16>(a, stream);
-  if (epi == EPI_F32 && a.C32) return launch_rows_epi<EPI_F32>(a, stream);
+  if (epi == EPI_ROWS && a.C32 && a.res) return launch_rows_epi<EPI_ROWS>(a, stream);
   return hipErrorInvalidValue;
 }
 

@@ -1245,7 +1245,7 @@ struct GptDecoder::Impl {
       a = g;
       a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.proj_w; a.ldw = kW; a.N = kW; a.bias = w.proj_b;
       a.res = xin; a.ldres = kW; a.C32 = xr; a.ldc32 = kW;
-      GPT_OK(launch_gemm_rows(a, EPI_F32, s));
+      GPT_OK(launch_gemm_rows(a, EPI_ROWS, s));
       xin = xr;
       GPT_OK(launch_gpt_ln_rows(xr, w.ln2_w, w.ln2_b, M, a16, lo, ovf, s));
       a = g;
@@ -1255,7 +1255,7 @@ struct GptDecoder::Impl {
       a = g;
       a.A = fc16; a.lda = kMLP; a.a_lo = fc_lo; a.K = kMLP; a.W = w.mp_w; a.ldw = kMLP; a.N = kW; a.bias = w.mp_b;
       a.res = xr; a.ldres = kW; a.C32 = xr; a.ldc32 = kW;
-      GPT_OK(launch_gemm_rows(a, EPI_F32, s));
+      GPT_OK(launch_gemm_rows(a, EPI_ROWS, s));
     }
   }
 

@@ -82,11 +82,27 @@ struct ActFilters {
 // a multiple of 64 (the 24- and 48-channel stages).
 constexpr int kActR = 16;
 
-template <bool OUT16>
-__global__ __launch_bounds__(256) void snake_aa_kernel(const float* __restrict__ x, ActFilters f,
-                                                       const float* __restrict__ alpha,
-                                                       const float* __restrict__ inv_beta, int T,
-                                                       int C, void* __restrict__ out, size_t out_lo) {
+// One activation of a launch; blockIdx.y picks it.
+struct ActCall {
+  const float* x;
+  void* out;
+  const float* alpha;
+  const float* inv_beta;
+  ActFilters f;
+};
+template <int G>
+struct ActGroup {
+  ActCall c[G];
+};
+
+template <bool OUT16, int G>
+__global__ __launch_bounds__(256) void snake_aa_kernel(ActGroup<G> grp, int T, int C, size_t out_lo) {
+  const ActCall& call = grp.c[G > 1 ? blockIdx.y : 0];
+  const float* __restrict__ x = call.x;
+  const ActFilters& f = call.f;
+  const float* __restrict__ alpha = call.alpha;
+  const float* __restrict__ inv_beta = call.inv_beta;
+  void* __restrict__ out = call.out;
   constexpr int R = kActR;
   constexpr int XW = R + 12;      // x window
   constexpr int ZW = 2 * R + 10;  // Z window: u = 2 t0 - 5 + i
@@ -198,6 +214,30 @@ __global__ __launch_bounds__(256) void conv_post_clamp_kernel(const float* __res
     for (int k = 0; k < 7; ++k) acc += as[(threadIdx.x + k) * RS + ic] * ws[ic * 7 + k];
   }
   wav[t] = fminf(1.0f, fmaxf(-1.0f, acc));
+}
+
+// g = v0 / 3 + v1 / 3 + v2 / 3 in EPI_RESAVG's order, and its f16 copy (a
+// split pair when lo is nonzero).  n a multiple of 4.
+__global__ __launch_bounds__(256) void avg3_kernel(const float4* __restrict__ v0, const float4* __restrict__ v1,
+                                                   const float4* __restrict__ v2, float4* __restrict__ g,
+                                                   half_t* __restrict__ g16, size_t lo, size_t n4) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const float4 a = v0[i], b = v1[i], c = v2[i];
+  auto mean = [](float x, float y, float z) { return ((0.f + x / 3.0f) + y / 3.0f) + z / 3.0f; };
+  const float m[4] = {mean(a.x, b.x, c.x), mean(a.y, b.y, c.y), mean(a.z, b.z, c.z), mean(a.w, b.w, c.w)};
+  g[i] = make_float4(m[0], m[1], m[2], m[3]);
+  if (!g16) return;
+  half_t h[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (lo)
+      split_f16(m[e], h[e], l[e]);
+    else
+      h[e] = (half_t)m[e];
+  }
+  *reinterpret_cast<half4*>(g16 + 4 * i) = half4{h[0], h[1], h[2], h[3]};
+  if (lo) *reinterpret_cast<half4*>(g16 + lo + 4 * i) = half4{l[0], l[1], l[2], l[3]};
 }
 
 __global__ void voc_f32_to_f16_kernel(const float* __restrict__ in, half_t* __restrict__ out,
@@ -406,7 +446,8 @@ struct Vocoder::Impl {
   void ensure(int T) {
     if (T <= cap) return;
     const size_t big = (size_t)T * 6144;  // C * T_s of every stage from the second on
-    const size_t need = 2 * ((size_t)T * 80 * 2 + (size_t)T * 1536 * 2 + 2 * big * 2) + 5 * big * 4 + 9 * 256;
+    // (the activations' operand, the convs1 output and the residual stream: one per resblock of a group)
+    const size_t need = 2 * ((size_t)T * 80 * 2 + (size_t)T * 1536 * 2 + 4 * big * 2) + 9 * big * 4 + 9 * 256;
     VOC_OK(hipStreamSynchronize(s));
     ws.reserve(need + 4096);
     mel16_lo = (size_t)T * 80;
@@ -414,11 +455,11 @@ struct Vocoder::Impl {
     a16_lo = g16_lo = big;
     mel16 = static_cast<half_t*>(ws.take(mel16_lo * 2 * 2));
     pre16 = static_cast<half_t*>(ws.take(pre16_lo * 2 * 2));
-    a16 = static_cast<half_t*>(ws.take(big * 2 * 2));
+    a16 = static_cast<half_t*>(ws.take(3 * big * 2 * 2));
     g16 = static_cast<half_t*>(ws.take(big * 2 * 2));
     x32 = static_cast<float*>(ws.take(big * 4));
-    h32 = static_cast<float*>(ws.take(big * 4));
-    t32 = static_cast<float*>(ws.take(big * 4));
+    h32 = static_cast<float*>(ws.take(3 * big * 4));
+    t32 = static_cast<float*>(ws.take(3 * big * 4));
     g32 = static_cast<float*>(ws.take(big * 4));
     act32 = static_cast<float*>(ws.take(big * 4));
     cap = T;
@@ -427,8 +468,9 @@ struct Vocoder::Impl {
   // ---------------------------------------------------------- launches
   // Conv of the f16 operand A (a split pair with lo at + a_lo); C16 (when
   // given) is a split pair buffer with lo at + c16_lo.
-  void conv(const Conv& c, const half_t* A, size_t a_lo, int T, int d, int pad, int epi, float* C32,
-            const float* res, float* C32b, half_t* C16, size_t c16_lo, int flag) {
+  GemmArgs conv_args(const Conv& c, const half_t* A, size_t a_lo, int T, int d, int pad, float* C32,
+                     const float* res, float* C32b = nullptr, half_t* C16 = nullptr, size_t c16_lo = 0,
+                     int flag = 0) const {
     GemmArgs g;
     if (f32) {
       g.split = c.scale ? 1 : 2;  // A split; W split too unless it holds v exactly
@@ -463,22 +505,33 @@ struct Vocoder::Impl {
     g.C16 = C16;
     g.ldc16 = c.n_out;
     g.flag = flag;
-    VOC_OK(launch_gemm(g, A_CONVP, (EpiMode)epi, s));
+    return g;
+  }
+  void conv(const Conv& c, const half_t* A, size_t a_lo, int T, int d, int pad, int epi, float* C32,
+            const float* res, float* C32b, half_t* C16, size_t c16_lo, int flag) {
+    VOC_OK(launch_gemm(conv_args(c, A, a_lo, T, d, pad, C32, res, C32b, C16, c16_lo, flag), A_CONVP, (EpiMode)epi, s));
   }
 
   // out16: out is a split pair buffer (lo at + out_lo, written in f32 mode).
-  void activation(const Act& a, const float* in, int T, void* out, bool out16, size_t out_lo = 0) {
+  // G activations of one width, each on its own input and output, in one launch.
+  template <int G>
+  void activations(const std::array<const Act*, G>& a, const std::array<const float*, G>& in,
+                   const std::array<void*, G>& out, int T, bool out16, size_t out_lo = 0) {
+    const int C = a[0]->C;
     // the kernel addresses the T x C activation with 32-bit byte offsets
-    if ((size_t)T * (size_t)a.C >= (size_t(1) << 29)) VOC_OK(hipErrorInvalidValue);
-    const size_t lanes = (size_t)((T + kActR - 1) / kActR) * a.C;
-    const dim3 grid((unsigned)((lanes + 255) / 256));
+    if ((size_t)T * (size_t)C >= (size_t(1) << 29)) VOC_OK(hipErrorInvalidValue);
+    const size_t lanes = (size_t)((T + kActR - 1) / kActR) * C;
+    const dim3 grid((unsigned)((lanes + 255) / 256), G);
+    ActGroup<G> g;
+    for (int i = 0; i < G; ++i) g.c[i] = {in[i], out[i], a[i]->alpha, a[i]->inv_beta, a[i]->filt};
     if (out16)
-      hipLaunchKernelGGL(snake_aa_kernel<true>, grid, dim3(256), 0, s, in, a.filt, a.alpha, a.inv_beta,
-                         T, a.C, out, f32 ? out_lo : 0);
+      hipLaunchKernelGGL((snake_aa_kernel<true, G>), grid, dim3(256), 0, s, g, T, C, f32 ? out_lo : 0);
     else
-      hipLaunchKernelGGL(snake_aa_kernel<false>, grid, dim3(256), 0, s, in, a.filt, a.alpha, a.inv_beta,
-                         T, a.C, out, (size_t)0);
+      hipLaunchKernelGGL((snake_aa_kernel<false, G>), grid, dim3(256), 0, s, g, T, C, (size_t)0);
     VOC_OK(hipGetLastError());
+  }
+  void activation(const Act& a, const float* in, int T, void* out, bool out16, size_t out_lo = 0) {
+    activations<1>({&a}, {in}, {out}, T, out16, out_lo);
   }
 
   // One resblock j over x [T][C]: three (act, dilated conv, act, conv, + res)
@@ -504,8 +557,51 @@ struct Vocoder::Impl {
 
   // Resblock group i over the upsampled x [T][C]: g = mean of the three
   // resblocks; g16o receives its f16 copy (the next upsampler's operand).
+  // The three run in step, each activation and each conv one launch for all
+  // of them (they do not depend on each other, and one alone leaves much of
+  // the chip idle); resblock r works in the r-th third of the buffers.
   void group(int i, const float* x, int T, float* g, half_t* g16o) {
-    for (int r = 0; r < 3; ++r) resblock(3 * i + r, x, T, nullptr, g, r > 0, r == 2 ? g16o : nullptr);
+    const int C = rb_channels(3 * i);
+    half_t* a[3];
+    float *t[3], *h[3];
+    for (int r = 0; r < 3; ++r) {
+      a[r] = a16 + (size_t)r * 2 * a16_lo;
+      t[r] = t32 + (size_t)r * a16_lo;
+      h[r] = h32 + (size_t)r * a16_lo;
+    }
+    const float* in[3] = {x, x, x};
+    bool in_step = true;  // the last convs too: else each adds to the mean in its epilogue
+    for (int pr = 0; pr < 3; ++pr) {
+      GemmArgs ga[3];
+      auto acts = [&](int which, const float* const (&src)[3]) {
+        activations<3>({&act[3 * i][2 * pr + which], &act[3 * i + 1][2 * pr + which], &act[3 * i + 2][2 * pr + which]},
+                       {src[0], src[1], src[2]}, {a[0], a[1], a[2]}, T, true, a16_lo);
+      };
+      acts(0, in);
+      const int d = kDil[pr];
+      for (int r = 0; r < 3; ++r)
+        ga[r] = conv_args(rb[3 * i + r][pr][0], a[r], a16_lo, T, d, (kRbKernel[r] - 1) * d / 2, t[r], nullptr);
+      VOC_OK(launch_gemm_group(ga, 3, A_CONVP, EPI_F32, s, &in_step));
+      const float* tc[3] = {t[0], t[1], t[2]};
+      acts(1, tc);
+      if (pr < 2 || in_step) {
+        for (int r = 0; r < 3; ++r)
+          ga[r] = conv_args(rb[3 * i + r][pr][1], a[r], a16_lo, T, 1, (kRbKernel[r] - 1) / 2, h[r], in[r]);
+        VOC_OK(launch_gemm_group(ga, 3, A_CONVP, EPI_F32, s));
+        for (int r = 0; r < 3; ++r) in[r] = h[r];
+      } else {
+        for (int r = 0; r < 3; ++r)
+          conv(rb[3 * i + r][pr][1], a[r], a16_lo, T, 1, (kRbKernel[r] - 1) / 2, EPI_RESAVG, nullptr, in[r], g,
+               r == 2 ? g16o : nullptr, g16_lo, r > 0);
+      }
+    }
+    if (in_step) {
+      const size_t n4 = (size_t)T * C / 4;
+      auto f4 = [](const float* p) { return reinterpret_cast<const float4*>(p); };
+      hipLaunchKernelGGL(avg3_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, f4(in[0]), f4(in[1]),
+                         f4(in[2]), reinterpret_cast<float4*>(g), g16o, f32 ? g16_lo : 0, n4);
+      VOC_OK(hipGetLastError());
+    }
   }
 
   void to_f16(const float* in, half_t* out, size_t n, size_t lo_off) {
