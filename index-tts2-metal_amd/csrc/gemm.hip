@@ -1627,6 +1627,13 @@ static hipError_t launch_tile(const GemmArgs& a, hipStream_t s) {
 // the k=5 conv 10.5 vs 15.5 us, w1|w3 5.2 vs 8.7, w2 5.9 vs 7.0.  Only the
 // tile shape changes, never the K split or the order of the MFMAs over K, so
 // a row's result is the same bits whichever tiling the batch gets.
+// The short-K ones (QKV, wo, res/skip: eight stages) keep four stages in
+// flight (a 5-stage ring): at M = 256 a decode step's 13 QKV, 14 wo-shaped and
+// 8 res/skip launches take 4.9, 7.2 and 4.3 us less than with three stages
+// (4: 0 to 2 less; 6: 3 to 5 less; all eight at once: no less), w1|w3 2.1 less
+// while its tiles are at most one a CU (28 more at 336 tiles).  The long-K
+// ones gain nothing.  The condition producer's split products, whose ring of
+// three holds 72 KB: a call of 24 codes 74.4 -> 69.4 us, of 553 96.3 -> 90.1.
 static bool few_tiles(const GemmArgs& a, int BM, int BN) {
   return (long)((a.M + BM - 1) / BM) * (a.N / BN) < 128;
 }
@@ -1809,7 +1816,7 @@ static hipError_t launch_split(const GemmArgs& a, hipStream_t s) {
     // The condition producer's products (M = a few hundred rows): 32-row
     // tiles when 64 x 64 leaves most CUs idle.  Its k=3 convs at 602 rows
     // (N = 512, K = 1536, both operands split): 9.8 vs 13.7 us per launch.
-    if (few_tiles(a, 64, 64)) return launch_tile<32, 64, 64, 3, AM, EPI, 2, 2, 1, SP>(a, s);
+    if (few_tiles(a, 64, 64)) return launch_tile<32, 64, 64, 5, AM, EPI, 2, 2, 1, SP>(a, s);
     return launch_tile<64, 64, 64, 3, AM, EPI, 2, 2, 1, SP>(a, s);
   }
 }
@@ -1834,7 +1841,10 @@ static hipError_t launch_am_epi(const GemmArgs& a, hipStream_t s) {
   }
   if constexpr (EPI == EPI_SWIGLU) {
     if (a.N % 192 == 0) {
-      if (few_tiles(a, 128, 192) && a.N % 128 == 0) return launch_tile<32, 128, 64, 3, AM, EPI, 2, 2>(a, s);
+      if (few_tiles(a, 128, 192) && a.N % 128 == 0) {
+        if (tile_count(a, 32, 128) <= 256) return launch_tile<32, 128, 64, 5, AM, EPI, 2, 2>(a, s);
+        return launch_tile<32, 128, 64, 3, AM, EPI, 2, 2>(a, s);
+      }
       return launch_tile<128, 192, 64, 3, AM, EPI, 4, 2>(a, s);
     }
   }
@@ -1865,7 +1875,7 @@ static hipError_t launch_am_epi(const GemmArgs& a, hipStream_t s) {
   }
   if constexpr (EPI == EPI_RESSKIP || EPI == EPI_DUAL) {
     if (a.N % 128 == 0) {
-      if (few_tiles(a, 64, 128)) return launch_tile<32, 64, 64, 3, AM, EPI, 2, 2>(a, s);
+      if (few_tiles(a, 64, 128)) return launch_tile<32, 64, 64, 5, AM, EPI, 2, 2>(a, s);
       return launch_tile<64, 128, 64, 3, AM, EPI, 2, 4>(a, s);
     }
   }
@@ -1883,7 +1893,7 @@ static hipError_t launch_am_epi(const GemmArgs& a, hipStream_t s) {
       return launch_tile<64, 64, 64, 3, AM, EPI, 2, 2, 2>(a, s);
     }
   }
-  if (few_tiles(a, 64, 64)) return launch_tile<32, 64, 64, 3, AM, EPI, 2, 2>(a, s);
+  if (few_tiles(a, 64, 64)) return launch_tile<32, 64, 64, 5, AM, EPI, 2, 2>(a, s);
   return launch_tile<64, 64, 64, 3, AM, EPI>(a, s);
 }
 
