@@ -596,6 +596,70 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
     pl[tid] = exp((double)(proc[lidx[tid]] - mx));
     ps[tid] = exp((double)(sv[p0 + tid] - mx));
   }
+  // the loop's bookkeeping (one thread)
+  auto record = [&](int next) {
+    st->argmax = next;
+    if (st->n_pred < st->max_pred) predicted[st->n_pred] = (uint32_t)next;
+    st->n_pred += 1;
+    if (next == kStop) {
+      st->stopped = 1;
+      st->stop_step = st->step;
+    } else {
+      if (st->n_in < st->max_pred + 1) inputs[st->n_in] = (uint32_t)next;
+      st->n_in += 1;
+      st->cur_token = next;
+    }
+    st->step += 1;
+  };
+  if (listed && m <= 64) {
+    // At most a wave of survivors (top-k 30): wave 0 takes them all.  The sums
+    // keep their order (every lane runs them, over LDS); what does not depend
+    // on them is a lane's work.  (Thread 0 alone, reading each survivor's score
+    // back from memory, took 12 us more of a code's 430.)
+    for (int i = tid; i < (N + 31) / 32; i += kSampleThreads) seen[i] = 0u;  // now: removed by top-p
+    __syncthreads();
+    if (tid >= 64) return;
+    const uint32_t idx = tid < m ? lidx[tid] : 0u;
+    const bool finite = tid < m && proc[idx] != -INFINITY;  // (ahead of top-p's stores)
+    if (use_p) {
+      double total = 0.0;
+      for (int q = 0; q < m; ++q) total += pl[q];
+      const double low_tail = 1.0 - (double)top_p;
+      if (tid < m) ps[tid] = ps[tid] / total;
+      __builtin_amdgcn_wave_barrier();
+      double cumulative = 0.0, mine = 0.0;
+      for (int p = 0; p < m; ++p) {
+        cumulative += ps[p];
+        mine = p == tid ? cumulative : mine;
+      }
+      if (tid < m - 1 && mine <= low_tail) {
+        const uint32_t i = si[p0 + tid];
+        proc[i] = -INFINITY;
+        atomicOr(&seen[i >> 5], 1u << (i & 31));
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    const bool keep = finite && !((seen[idx >> 5] >> (idx & 31)) & 1u);
+    const uint64_t kept = __ballot(keep);
+    double total = 0.0;
+    for (int q = 0; q < m; ++q)
+      if ((kept >> q) & 1ull) total += pl[q];
+    uint64_t rng = st->rng;
+    const double target = sm64_unit(rng) * total;
+    double cumulative = 0.0;
+    int last = -1, pick = -1;
+    for (int q = 0; q < m && pick < 0; ++q) {
+      if (!((kept >> q) & 1ull) || pl[q] <= 0.0) continue;
+      last = q;
+      cumulative += pl[q];
+      if (target < cumulative) pick = q;
+    }
+    if (tid != 0) return;
+    st->rng = rng;
+    const int at = pick < 0 ? last : pick;
+    record(at < 0 ? 0 : (int)lidx[at]);
+    return;
+  }
   __syncthreads();
   if (tid != 0) return;
   // survivors in index order: (index, its exp) -- removed ones are skipped
@@ -635,19 +699,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
     cumulative += pr;
     if (target < cumulative) pick = i;
   });
-  const int next = (int)(pick == 0xffffffffu ? last : pick);
-  st->argmax = next;
-  if (st->n_pred < st->max_pred) predicted[st->n_pred] = (uint32_t)next;
-  st->n_pred += 1;
-  if (next == kStop) {
-    st->stopped = 1;
-    st->stop_step = st->step;
-  } else {
-    if (st->n_in < st->max_pred + 1) inputs[st->n_in] = (uint32_t)next;
-    st->n_in += 1;
-    st->cur_token = next;
-  }
-  st->step += 1;
+  record((int)(pick == 0xffffffffu ? last : pick));
 }
 
 // argmax_row (gpt.cpp:1297-1308), second stage: the first maximum over the

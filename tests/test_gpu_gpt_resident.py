@@ -166,3 +166,20 @@ def test_decode_values_past_f16(mit2, tensors, monkeypatch, where):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("top_k,top_p", [(1, 0.5), (2, 1.0), (30, 0.8), (30, 1.0), (30, 0.05), (63, 0.9), (64, 0.9),
+                                         (65, 0.9), (200, 0.99)])
+def test_sampler_survivor_counts(pair2, orc, mit2, top_k, top_p):
+    """The sampler's wave form (up to 64 survivors) and the general form next to
+    it, against the oracle's processors on the same logits: the same tokens kept
+    and, drawn from them, the same code."""
+    x = _rows(15, 100 + top_k)
+    cfg = dict(temperature=0.9, top_k=top_k, top_p=top_p, repetition_penalty=1.5)
+    g = orc.GPT(_tensors(mit2, {}, 2))
+    for seed in range(3):
+        got = pair2[1].gpt_kv_sample(x, 6, seed, **cfg)
+        ref = g.kv_sample(x, 6, seed, **cfg)
+        assert got["predicted"].tolist() == ref["predicted"].tolist()
+        a, b = got["last_processed_logits"], ref["last_processed_logits"]
+        assert np.array_equal(np.isfinite(a), np.isfinite(b))
