@@ -66,9 +66,9 @@ BENCH_PMC = ("python3 -u bench.py --steps 1 --warmup 1 --no-cpu-baseline --no-cp
 GPT_BENCH = ("python3 -u bench.py --steps 1 --warmup 1 --no-cpu-baseline --no-configs --kernel-launches 5 "
              "--voc-calls 0 --acoustic-calls 0 --cond-calls 1")
 GPT_CMDS = [
-    f"MIT2CFM_GRAPH=0 rocprofv3 --kernel-trace --stats -T --output-format csv -d $RAW/gpttrace -o bench -- {GPT_BENCH}",
-    f"MIT2CFM_GRAPH=0 rocprofv3 --pmc FETCH_SIZE -T --output-format csv -d $RAW/gptpmc_fetch -o fetch -- {GPT_BENCH}",
-    f"MIT2CFM_GRAPH=0 rocprofv3 --pmc WRITE_SIZE -T --output-format csv -d $RAW/gptpmc_write -o write -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --kernel-trace --stats -T --output-format csv -d $RAW/gpttrace -o bench -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --pmc FETCH_SIZE -T --output-format csv -d $RAW/gptpmc_fetch -o fetch -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --pmc WRITE_SIZE -T --output-format csv -d $RAW/gptpmc_write -o write -- {GPT_BENCH}",
 ]
 
 
@@ -591,12 +591,11 @@ def gemv_roles(rows: list[dict], grid_key: str, wg_key: str) -> dict:
     within a layer (c_attn, the attention, attn c_proj, c_fc, mlp c_proj):
     two products can share a grid, so the grid alone does not name them.
     `rows` are dispatches in launch order."""
-    g = [r for r in rows if "gemv_kernel" in r["Kernel_Name"] and "gemv_rows" not in r["Kernel_Name"]]
+    g = [r for r in rows if "gemv_kernel" in r["Kernel_Name"]]
     roles = {}
     # attn c_proj is the GEMV launched right after an attention combine; the
     # first layer where the pattern is whole names all four
-    seq = [r for r in rows if any(k in r["Kernel_Name"] for k in ("gemv_kernel", "attn_combine_kernel"))
-           and "gemv_rows" not in r["Kernel_Name"]]
+    seq = [r for r in rows if any(k in r["Kernel_Name"] for k in ("gemv_kernel", "attn_combine_kernel"))]
     for i in range(len(seq) - 3):
         if "attn_combine_kernel" in seq[i]["Kernel_Name"] and all("gemv_kernel" in seq[i + k]["Kernel_Name"]
                                                                    for k in (1, 2, 3)):
@@ -615,12 +614,12 @@ def gemv_roles(rows: list[dict], grid_key: str, wg_key: str) -> dict:
 
 def gpt_kernel_key(r: dict, roles: dict) -> str:
     n = r["Kernel_Name"]
-    for k in ("gemv_rows_kernel", "gemv_kernel", "attn_split_kernel", "attn_combine_kernel", "sample_kernel",
+    for k in ("gemv_kernel", "attn_split_kernel", "attn_combine_kernel", "sample_kernel",
               "embed_rows_kernel", "embed_kernel", "argmax_kernel", "advance_rows_kernel"):
         if k in n:
             if k.startswith("gemv"):
                 blocks = int(r["Grid_Size_X"]) // int(r["Workgroup_Size_X"])
-                role = roles.get(r["Kernel_Id"]) if k == "gemv_kernel" else "prefill"
+                role = roles.get(r["Kernel_Id"])
                 return f"{k} {role or '?'} (grid {blocks}x{r['Workgroup_Size_X']})"
             return k
     return n[:40]
@@ -660,7 +659,7 @@ def write_gpt_profiles(raw: Path, out: Path) -> None:
     cmds = "\n".join(GPT_CMDS)
     md = f"""# GPT mel-code decoder: 553 codes after a 150-row prefix, 24 layers -- rocprofv3 kernel trace
 
-Commands (repo root, MI355X, one GPU).  The HIP-graph replay is switched off with MIT2CFM_GRAPH=0
+Commands (repo root, MI355X, one GPU).  The HIP-graph replay is switched off with MIT2CFM_GRAPH=0, the resident step kernel with MIT2CFM_GPT_RESIDENT=0
 (every kernel launched directly; the same kernels): one earlier kernel-trace run with graph replay
 ended in a host SIGSEGV inside hipGraphLaunch of the GPT step graph.
 
