@@ -5,8 +5,8 @@ tiles chosen by the rows, and their mean is taken by a kernel of its own.
 A group's output must equal, bit for bit, the mean of its resblocks run one by
 one: the tiles and the launch change no sum's order, and the mean is
 ((0 + v0 / 3) + v1 / 3) + v2 / 3 in fp32 either way.  Row counts sit at the edges
-of the tile rules (64-row tiles of the 768- and 384-channel stages: up to 32,
-64, 100 tiles; the pipelined 128-row tiles from 128 to 256, whose convs run one
+of the tile rules (64-row tiles of the 768- and 384-channel stages: up to 40, 64,
+90, 100 tiles; the pipelined 128-row tiles from 128 to 256, whose convs run one
 by one, and beyond), odd counts and one row among them.
 """
 from __future__ import annotations
@@ -24,8 +24,8 @@ def ctx_bvg(mit2, tensors):
     c.close()
 
 
-CASES = [(0, t) for t in (1, 17, 320, 321, 640, 641, 1024, 1025, 2752, 5504)]
-CASES += [(1, t) for t in (64, 640, 641, 1345, 2112, 5441)]
+CASES = [(0, t) for t in (1, 17, 320, 384, 385, 640, 641, 960, 1024, 1025, 2752, 5504)]
+CASES += [(1, t) for t in (64, 832, 833, 1345, 1921, 2112, 5441)]
 CASES += [(2, 65), (2, 16385), (3, 127), (4, 255), (4, 33001), (5, 511)]
 
 
