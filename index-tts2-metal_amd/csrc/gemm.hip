@@ -1763,33 +1763,15 @@ static bool launch_conv_window(const GemmArgs& a0, hipStream_t s, hipError_t& e)
 }
 
 // The wide convs of a short call (a few hundred rows): smaller tiles than
-// 64 x 128, so that more CUs take part, and K split over two or four wave
-// groups of the workgroup, as the time is the latency of the K stages (up to
-// 132).  Whole calls, us, at 20 / 61 / 120 / 180 frames:
-//  f16   64 x 128 1358 / 1537 / 1746 / 1903; 32 x 64, one group 1209 / 1336 /
-//        1556 / 1814; two groups 986 / 1129 / 1416 / 1711; four (two where K
-//        does not divide) 934 / 1077 / 1453 / 1805
-//  f32   1700 / 1908 / 2077 / 2350; one group 1442 / 1627 / 1898 / 2295; two
-//        1197 / 1429 / 1999 / 2416; four 1180 / 1417 / 1992 / 2403
-// (the K split is by rows here, so a conv's rounding differs between short
-// and long calls; within a call a group and its resblocks alone agree).
+// 64 x 128, so that more CUs take part; the time is the latency of the K stages.
 template <int EPI, int SP>
 static bool launch_conv_rows(const GemmArgs& a, hipStream_t s, hipError_t& e) {
   if (a.N % 128 != 0 || a.row_nb != 0) return false;
   const long t = tile_count(a, 64, 128);
-  const int stages = a.K / 64;
-  if constexpr (SP < 2) {
-    const bool groups = t <= 40 || (SP == 0 ? t <= 90 : a.N < 768 && t <= 64);
-    if (t <= 40 && stages % 4 == 0) {
-      e = launch_tile<32, 64, 64, SP == 0 ? 3 : 2, A_CONVP, EPI, 2, 2, 4, SP>(a, s);
-      return true;
-    }
-    if (groups && stages % 2 == 0) {
-      e = launch_tile<32, 64, 64, 3, A_CONVP, EPI, 2, 2, 2, SP>(a, s);
-      return true;
-    }
-  }
-  if (t <= 64) {
+  constexpr int kDeep = SP == 0 ? 6 : SP == 1 ? 5 : 3;  // stages that leave room for two workgroups a CU
+  if (t <= 32) {
+    e = launch_tile<32, 64, 64, kDeep, A_CONVP, EPI, 2, 2, 1, SP>(a, s);
+  } else if (t <= 64) {
     e = launch_tile<32, 64, 64, 3, A_CONVP, EPI, 2, 2, 1, SP>(a, s);
   } else if (t <= 100 && SP < 2) {
     e = launch_tile<64, 64, 64, SP == 0 ? 4 : 3, A_CONVP, EPI, 4, 2, 1, SP>(a, s);
@@ -1822,7 +1804,7 @@ static hipError_t launch_split(const GemmArgs& a, hipStream_t s) {
         return launch_tile<64, 96, 64, 3, AM, EPI, 4, 1, 1, SP>(a, s);
       }
     }
-    if constexpr (EPI == EPI_F32 || EPI == EPI_RESAVG) {
+    if constexpr (EPI == EPI_F32) {
       hipError_t e;
       if (launch_conv_rows<EPI, SP>(a, s, e)) return e;
     }
@@ -1848,7 +1830,7 @@ static hipError_t launch_am_epi(const GemmArgs& a, hipStream_t s) {
       hipError_t e;
       if (a.conv_window && a.M == a.T && a.row_nb == 0 && launch_conv_window<EPI, 0>(a, s, e)) return e;
     }
-    if constexpr (EPI == EPI_F32 || EPI == EPI_RESAVG) {
+    if constexpr (EPI == EPI_F32) {
       hipError_t e;
       if (launch_conv_rows<EPI, 0>(a, s, e)) return e;
     }
