@@ -231,9 +231,10 @@ hipError_t launch_gemm_group(const GemmArgs* a, int n, AMode amode, EpiMode epi,
 
 // The GPT prefill's products: A_PLAIN with a split A and an f16-exact W
 // (GemmArgs::split = 1), epilogue EPI_KVCACHE, EPI_GELU16 or EPI_ROWS.  K a
-// multiple of 256, N of 64.  Each K stage is summed by itself before it joins
-// the total (over the whole stack an error against float64 of 3.6e-7, as the
-// vector units gave; 7e-7 as one chain).
+// multiple of 1280 (four quarters of whole blocks of five K stages), N of 64.
+// Each K stage is summed by itself before it joins a block, a quarter and the
+// total, in one order for every tile (as one chain over K the stack's error
+// against float64 doubled, 3.6e-7 to 7e-7).
 hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream);
 
 }  // namespace mit2hip

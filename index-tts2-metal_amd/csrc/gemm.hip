@@ -603,17 +603,24 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
       for (int j = 0; j < NI; ++j) accx[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  // The GPT prefill's long sums: each stage's product is summed by itself and
-  // added to a partial sum, and that to the total every eight stages, so no
-  // value passes through a chain of K / 32 matrix-core additions.
+  // The GPT prefill's long sums.  Each stage's product is summed by itself and
+  // added to a block of kFoldStages stages, the blocks in order to their
+  // quarter of K (the lo products of a quarter join it as one chain), and the
+  // quarters in pairs: (0 + 1) + (2 + 3).  So no value passes through a chain of
+  // K / 32 matrix-core additions, and the order is the same for one, two and
+  // four K groups: a row's bits do not depend on which tile its call takes.
   constexpr bool kFold = EPI == EPI_ROWS || EPI == EPI_GELU16 || EPI == EPI_KVCACHE;
-  static_assert(!kFold || SP == 1, "the GPT prefill's operands");
-  floatx4 tot[kFold ? MI : 1][kFold ? NI : 1], tot8[kFold ? MI : 1][kFold ? NI : 1];
+  constexpr int kFoldStages = 5;
+  static_assert(!kFold || (SP == 1 && PIPE == 0 && KG <= 4 && KG != 3), "the GPT prefill's operands");
+  floatx4 blk[kFold ? MI : 1][kFold ? NI : 1], part[kFold ? MI : 1][kFold ? NI : 1];
+  floatx4 pair[kFold ? MI : 1][kFold ? NI : 1], half[kFold ? MI : 1][kFold ? NI : 1];
+  int fold_left = kFoldStages, part_left = kFold ? KT * KG / 4 : 0, parts = 0;  // (wave-uniform)
   if constexpr (kFold) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) tot[i][j] = tot8[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NI; ++j)
+        blk[i][j] = part[i][j] = pair[i][j] = half[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
   // Fragment reads.  Every fragment row of this lane has the same swizzle
@@ -684,21 +691,36 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
       }
     }
     if constexpr (kFold) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) {
-          tot8[i][j] += acc[i][j];
-          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-      if ((kt & 7) == 7) {
+      auto each = [&](auto f) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < NI; ++j) {
-            tot[i][j] += tot8[i][j];
-            tot8[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-          }
+          for (int j = 0; j < NI; ++j) f(i, j);
+      };
+      constexpr floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+      each([&](int i, int j) {
+        blk[i][j] += acc[i][j];
+        acc[i][j] = zero;
+      });
+      if (--fold_left == 0) {
+        fold_left = kFoldStages;
+        each([&](int i, int j) {
+          part[i][j] += blk[i][j];
+          blk[i][j] = zero;
+        });
+      }
+      if (--part_left == 0) {
+        part_left = KT * KG / 4;
+        ++parts;
+        each([&](int i, int j) {
+          pair[i][j] += part[i][j] + accx[i][j] * kSplitInv;
+          part[i][j] = accx[i][j] = zero;
+        });
+        if (KG == 1 && parts == 2)
+          each([&](int i, int j) {
+            half[i][j] = pair[i][j];
+            pair[i][j] = zero;
+          });
       }
     }
   };
@@ -893,9 +915,9 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j] + tot8[i][j];
+      for (int j = 0; j < NI; ++j) acc[i][j] = KG == 1 ? half[i][j] + pair[i][j] : pair[i][j];
   }
-  if constexpr (SP > 0) {
+  if constexpr (SP > 0 && !kFold) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -935,13 +957,23 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
     wait_lgkmcnt0();
     __syncthreads();
     if (kg > 0) return;
-#pragma unroll
-    for (int g = 1; g < KG; ++g) {
-      const floatx4* red = red_buf(g);
+    if constexpr (kFold && KG == 4) {  // the quarters in pairs
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] += red[((wave * MI + i) * NI + j) * 64 + lane];
+        for (int j = 0; j < NI; ++j) {
+          const int at = ((wave * MI + i) * NI + j) * 64 + lane;
+          acc[i][j] = (acc[i][j] + red_buf(1)[at]) + (red_buf(2)[at] + red_buf(3)[at]);
+        }
+    } else {
+#pragma unroll
+      for (int g = 1; g < KG; ++g) {
+        const floatx4* red = red_buf(g);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] += red[((wave * MI + i) * NI + j) * 64 + lane];
+      }
     }
   }
 
@@ -2071,7 +2103,7 @@ static hipError_t launch_rows_epi(const GemmArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream) {
-  if (!gemm_spans_fit(a, A_PLAIN) || a.split != 1 || a.a_lo == 0 || !a.A || !a.W || !a.bias || a.K % 256 != 0 ||
+  if (!gemm_spans_fit(a, A_PLAIN) || a.split != 1 || a.a_lo == 0 || !a.A || !a.W || !a.bias || a.K % 1280 != 0 ||
       a.N % 64 != 0 || a.row_nb != 0 || a.n_store != 0 || a.colperm || a.lda < a.K || a.ldw < a.K)
     return hipErrorInvalidValue;
   if (epi == EPI_KVCACHE && a.N == 3 * kGptW && a.C32 && a.C32b && a.C32c && a.T >= 0 && a.T + a.M <= a.Tpad)

@@ -58,6 +58,33 @@ def test_prefill_equals_row_prefill(ctx2, monkeypatch, M):
     assert max(errs) <= 1e-5 and got[3] == ref[3]
 
 
+def test_a_row_does_not_depend_on_the_prefix_length(mit2, tensors):
+    """The tiles and K groups of the products follow the row count; a row's bits
+    do not.  One layer whose last row attends to itself alone: keys are 8 x the
+    queries' weights, and the rows before it are its negative, hundreds of units
+    of score below, probability exactly 0.  So its value, projection and MLP are
+    the same sums whatever stands before it."""
+    t = dict(mit2.synthetic_gpt_tensors(layers=1))
+    w = np.array(t["gpt.gpt.h.0.attn.c_attn.weight"], np.float32).reshape(W, 3 * W)
+    b = np.array(t["gpt.gpt.h.0.attn.c_attn.bias"], np.float32)
+    w[:, :W] *= 8
+    w[:, W : 2 * W] = w[:, :W]
+    b[: 2 * W] = 0
+    t["gpt.gpt.h.0.attn.c_attn.weight"], t["gpt.gpt.h.0.attn.c_attn.bias"] = w, b
+    x = _rows(1, 77)
+    c = mit2.Context({**tensors, **t}, device=0)
+    try:
+        ref = None
+        for M in (1, 2, 16, 33, 64, 65, 128, 129, 193, 213, 257, 385, 450, 833, 1024, 1025, 1100):
+            print(f"row bits M={M}", flush=True)
+            got = c.gpt_cached_decode(np.concatenate([np.repeat(-x, M - 1, 0), x]), M - 1)
+            ref = got if ref is None else ref
+            for a, r in zip(got[:3], ref[:3]):
+                assert np.isfinite(a).all() and np.array_equal(a, r)
+    finally:
+        c.close()
+
+
 def test_prefill_caches_serve_the_decode(ctx2, monkeypatch):
     """Tokens decoded after the prefill read the caches it wrote."""
     prefix = _rows(97, 5)
