@@ -27,8 +27,9 @@
 //
 // A step normally runs as one resident kernel (gpt_token.hip); the kernels
 // below are its plain form, fp32 throughout, one launch a product: for values
-// past f16's range, for a GPU that cannot hold all of that kernel's workgroups
-// at once, and for rows prefilled one by one.
+// past f16's range and for a GPU that cannot hold all of that kernel's
+// workgroups at once; past f16's range the prefix goes in chunks of 8 rows
+// through their multi-row form.
 //
 // Every matrix-vector product reads its weights from HBM: each once per
 // step (f16, 0.98 GB for 24 layers) and used for one multiply-add.  The GEMV
@@ -79,6 +80,7 @@ constexpr int kStart = (int)GptDecoder::kStartToken, kStop = (int)GptDecoder::kS
 constexpr int kChunk = GPT_ATTN_KEYS;  // keys per attention split
 static_assert(kChunk % 64 == 0 && kChunk <= 512, "a split is whole passes of 64 keys, one score per thread");
 constexpr int kStepsPerCheck = 8;  // decode steps replayed between stop-flag reads
+constexpr int kPlainRows = 8;       // prefix rows per chunk of the plain (fp32) prefill
 constexpr int kPrefillRows = 1024;  // most prefix rows per prefill chunk (36 KB of workspace a row)
 
 enum { PRO_PLAIN = 0, PRO_LN = 1, PRO_LN2 = 2 };
@@ -292,6 +294,113 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
       a.blk_val[blockIdx.x] = bv;
       a.blk_idx[blockIdx.x] = bi;
     }
+  }
+}
+
+// The plain prefill's multi-row form of gemv_kernel: y[m] = W pro(x[m]) + b for
+// the rows m < mrows = min(kPlainRows, pend - kv) of a prefix chunk (rows kv..),
+// so each weight row is read once per chunk instead of once per prefix row.
+// The chunk's inputs (normalised first, for the LayerNorm prologue) are
+// staged in LDS; every sum runs in gemv_kernel's order (the same lane
+// layout, the same two partial sums, the same group reduction and the same
+// LayerNorm statistics), so a prefix row gets the same values either way.
+template <int K, int LPR, int WAVES, int PRO, int EPI>
+__global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
+  constexpr int MR = kPlainRows;
+  constexpr int RPW = 64 / LPR;
+  constexpr int CH = K / (8 * LPR);
+  constexpr int ROWS = WAVES * RPW;
+  static_assert(K % (8 * LPR) == 0, "K must be a multiple of 8 * LPR");
+  static_assert(PRO != PRO_LN2 && EPI != EPI_LOGITS, "the prefill has no head");
+  static_assert(PRO == PRO_PLAIN || K == kW, "LayerNorm prologues take the 1280-wide stream");
+  __shared__ float4 xs[MR][K / 4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int sub = lane / LPR, j = lane % LPR;
+  const int kv = a.st->kv;
+  const int mrows = min(MR, a.st->pend - kv);
+  const int r = blockIdx.x * ROWS + wave * RPW + sub;
+
+  half8 w[CH];
+  {
+    const half8* src = reinterpret_cast<const half8*>(a.w + (size_t)min(r, a.N - 1) * K) + j;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) w[c] = src[c * LPR];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // stage the chunk's inputs (rows past mrows are zeros)
+  if constexpr (PRO == PRO_PLAIN) {
+    for (int i = threadIdx.x; i < MR * (K / 4); i += WAVES * 64) {
+      const int mm = i / (K / 4), k4 = i % (K / 4);
+      xs[mm][k4] = mm < mrows ? reinterpret_cast<const float4*>(a.x + (size_t)mm * K)[k4]
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  } else {
+    // one wave per row, lanes laid out as a 32-lane group (both halves
+    // compute the same values; the first half stores them)
+    constexpr int CH32 = K / (8 * 32);
+    const int jj = lane & 31;
+    for (int mm = wave; mm < MR; mm += WAVES) {
+      float v[CH32][8];
+      if (mm < mrows) {
+        float g[CH32][8], b[CH32][8];
+        load_chunks<32, CH32>(v, a.x + (size_t)mm * K, jj);
+        load_chunks<32, CH32>(g, a.g1, jj);
+        load_chunks<32, CH32>(b, a.b1, jj);
+        group_layernorm<32, CH32>(v, g, b);
+      } else {
+#pragma unroll
+        for (int c = 0; c < CH32; ++c)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[c][e] = 0.f;
+      }
+      if (lane < 32) {
+#pragma unroll
+        for (int c = 0; c < CH32; ++c) {
+          xs[mm][2 * (jj + 32 * c)] = make_float4(v[c][0], v[c][1], v[c][2], v[c][3]);
+          xs[mm][2 * (jj + 32 * c) + 1] = make_float4(v[c][4], v[c][5], v[c][6], v[c][7]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  float wf[CH][8];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wf[c][e] = (float)w[c][e];
+  // one chunk row at a time (hoisting every row's LDS reads costs registers)
+#pragma unroll
+  for (int mm = 0; mm < MR; ++mm) {
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int q4 = 2 * (j + c * LPR);
+      const float4 lo = xs[mm][q4], hi = xs[mm][q4 + 1];
+      s0 += wf[c][0] * lo.x; s1 += wf[c][1] * lo.y;
+      s0 += wf[c][2] * lo.z; s1 += wf[c][3] * lo.w;
+      s0 += wf[c][4] * hi.x; s1 += wf[c][5] * hi.y;
+      s0 += wf[c][6] * hi.z; s1 += wf[c][7] * hi.w;
+    }
+    const float acc = group_sum<LPR>(s0 + s1);
+    if (j == 0 && r < a.N && mm < mrows) {
+      const float v = acc + a.bias[r];
+      if constexpr (EPI == EPI_GELU) {
+        a.y[(size_t)mm * a.N + r] = gelu_new(v);
+      } else if constexpr (EPI == EPI_RES) {
+        a.y[(size_t)mm * a.N + r] += v;
+      } else {
+        if (r < kW) {
+          a.q[(size_t)mm * kW + r] = v;
+        } else if (kv + mm < a.st->cap) {
+          const int c = r - (r < 2 * kW ? kW : 2 * kW);  // head c / 64, dim c % 64
+          float* cache = r < 2 * kW ? a.kc : a.vc;
+          cache[((size_t)(c >> 6) * a.st->cap + kv + mm) * kHD + (c & 63)] = v;
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -702,6 +811,18 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
   record((int)(pick == 0xffffffffu ? last : pick));
 }
 
+// Rows kv .. kv + mrows - 1 of the prefix into the chunk buffer.
+__global__ __launch_bounds__(256) void embed_rows_kernel(const GptState* st, const float* rows, float* x) {
+  const int mrows = min(kPlainRows, st->pend - st->kv);
+  const float4* src = reinterpret_cast<const float4*>(rows + (size_t)st->kv * kW);
+  for (int i = threadIdx.x; i < mrows * (kW / 4); i += 256) reinterpret_cast<float4*>(x)[i] = src[i];
+}
+
+// The chunk is done: its rows join the caches.
+__global__ void advance_rows_kernel(GptState* st) {
+  st->kv += max(0, min(kPlainRows, st->pend - st->kv));
+}
+
 // argmax_row (gpt.cpp:1297-1308), second stage: the first maximum over the
 // head blocks' maxima (ties go to the lower row), then the bookkeeping of the
 // loop of run_gpt_kv_greedy_cpu (gpt.cpp:1890-1909): record the prediction,
@@ -780,30 +901,32 @@ __global__ __launch_bounds__(320) void embed_kernel(const GptState* st, const fl
 // gpt.cpp:1147-1170, with cpu_attention_single_query, tokenizer_tests.cpp:
 // 4034-4060) over the st->kv + 1 cache rows (the current row included: the
 // c_attn kernel already wrote it), in two launches with no waiting between
-// blocks.  attn_split_kernel: block (head h, split s) takes keys
+// blocks.  attn_split_kernel: block (head h, split s, query row z) takes keys
 // 256 s .. 256 s + 255 -- all of its key and value loads issued together
 // (the kernel is latency-bound) -- and writes the split's max m_s, sum
 // l_s = sum exp(score - m_s) and unnormalised output sum exp(score - m_s) v;
 // a head with a single split writes its output directly.  attn_combine_kernel
 // merges the splits: out = sum_s e^(m_s - M) o_s / sum_s e^(m_s - M) l_s with
 // M = max m_s (eight splits per round trip, rescaled when M grows).  Scores: 8 lanes per key, 8 dims each; the output: 16 lanes
-// per key, 4 dims each.
+// per key, 4 dims each.  z is the query row of a prefill chunk (row z sees
+// the keys up to its own position kv + z); a decode step has one query.
 constexpr int kAttnThreads = 512;
 constexpr int kPartF = 2 + kHD;  // per split: max, sum, unnormalised output
 
 // What an attention block needs from the state: whether it has nothing to do
-// (the decode stopped, or the caches have no rows) and its key count.  The
-// three fields are read before anything is decided, and all of them decide,
-// so the loads are issued together and their latencies overlap; tested one
-// after another (as short-circuit tests with the key count read after them),
-// each load waited for the one before.
+// (the decode stopped, row z is past the prefill chunk, or the caches have
+// no rows) and row z's key count.  The four fields are read before anything
+// is decided, and all of them decide, so the loads are issued together and
+// their latencies overlap; tested one after another (as short-circuit tests
+// with the key count read after them), each load waited for the one before.
 struct AttnRow {
   bool idle;
   int keys;
 };
-__device__ __forceinline__ AttnRow attn_row(const GptState* st, int check_stop) {
-  const int kv = st->kv, stopped = st->stopped, cap = st->cap;
-  return {(check_stop && stopped) || cap <= 0, min(kv + 1, cap)};
+__device__ __forceinline__ AttnRow attn_row(const GptState* st, int z, int check_stop) {
+  const int kv = st->kv, stopped = st->stopped, cap = st->cap, pend = st->pend;
+  const bool live = gridDim.z == 1 || z < min((int)gridDim.z, pend - kv);
+  return {(check_stop && stopped) || !live || cap <= 0, min(kv + z + 1, cap)};
 }
 
 __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q, const float* kc, const float* vc,
@@ -813,12 +936,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
   constexpr int kKeysPerPass = kAttnThreads / 8, kPass = kChunk / kKeysPerPass;
   constexpr int kVKeysPerPass = kAttnThreads / 16, kVPass = kChunk / kVKeysPerPass;
   constexpr int kGroups = kAttnThreads / 16;  // output key groups
-  const int h = blockIdx.x, sp = blockIdx.y, tid = threadIdx.x;
-  const AttnRow row = attn_row(st, check_stop);
+  const int h = blockIdx.x, sp = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
+  const AttnRow row = attn_row(st, z, check_stop);
   if (row.idle) return;
   const int kvn = row.keys;
   const int nsplit = (kvn + kChunk - 1) / kChunk;
   if (sp >= nsplit) return;
+  q += (size_t)z * kW;
   const int t0 = sp * kChunk, n = min(kChunk, kvn - t0), last = kvn - 1;
   __shared__ float sc[kChunk];
   __shared__ float4 red[kGroups][kHD / 4];
@@ -884,9 +1008,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
 #pragma unroll
     for (int gg = 0; gg < kGroups; ++gg) od += reinterpret_cast<const float*>(&red[gg][0])[tid];
     if (nsplit == 1) {
-      out[h * kHD + tid] = od / l;
+      out[(size_t)z * kW + h * kHD + tid] = od / l;
     } else {
-      float* pp = part + ((size_t)h * nsplit_max + sp) * kPartF;
+      float* pp = part + (((size_t)z * kHeads + h) * nsplit_max + sp) * kPartF;
       pp[2 + tid] = od;
       if (tid == 0) { pp[0] = m; pp[1] = l; }
     }
@@ -895,12 +1019,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(const float* q
 
 __global__ __launch_bounds__(64) void attn_combine_kernel(const GptState* st, const float* part, float* out,
                                                           int nsplit_max, int check_stop) {
-  const int h = blockIdx.x, d = threadIdx.x;
-  const AttnRow row = attn_row(st, check_stop);
+  const int h = blockIdx.x, z = blockIdx.z, d = threadIdx.x;
+  const AttnRow row = attn_row(st, z, check_stop);
   if (row.idle) return;
   const int nsplit = (row.keys + kChunk - 1) / kChunk;
   if (nsplit == 1) return;  // written by the split kernel
-  const float* ph = part + (size_t)h * nsplit_max * kPartF;
+  const float* ph = part + ((size_t)z * kHeads + h) * nsplit_max * kPartF;
   // eight splits per round trip (the loads are issued before they are used)
   float M = -INFINITY, L = 0.f, O = 0.f;
   for (int s0 = 0; s0 < nsplit; s0 += 8) {
@@ -929,7 +1053,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const GptState* st, co
     }
     M = Mn;
   }
-  out[h * kHD + d] = O / L;
+  out[(size_t)z * kW + h * kHD + d] = O / L;
 }
 
 // Launch shapes: rows per block = WAVES * (64 / LPR) * UR.
@@ -971,6 +1095,18 @@ void launch_attn_proj(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_PR
 void launch_fc(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_FC_SHAPE, PRO_LN, EPI_GELU>(a, s); }
 void launch_mlp_proj(const GemvArgs& a, hipStream_t s) { launch_gemv<kMLP, GPT_MP_SHAPE, PRO_PLAIN, EPI_RES>(a, s); }
 void launch_head(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_HEAD_SHAPE, PRO_LN2, EPI_LOGITS>(a, s); }
+
+// The plain prefill chunk's GEMVs (lanes per row, waves per block).
+template <int K, int LPR, int WAVES, int PRO, int EPI>
+void launch_rows(const GemvArgs& a, hipStream_t s) {
+  constexpr int rows = WAVES * (64 / LPR);
+  hipLaunchKernelGGL((gemv_rows_kernel<K, LPR, WAVES, PRO, EPI>), dim3((a.N + rows - 1) / rows), dim3(WAVES * 64), 0,
+                     s, a);
+}
+void launch_qkv_rows(const GemvArgs& a, hipStream_t s) { launch_rows<kW, 32, 4, PRO_LN, EPI_QKV>(a, s); }
+void launch_attn_proj_rows(const GemvArgs& a, hipStream_t s) { launch_rows<kW, 32, 4, PRO_PLAIN, EPI_RES>(a, s); }
+void launch_fc_rows(const GemvArgs& a, hipStream_t s) { launch_rows<kW, 32, 4, PRO_LN, EPI_GELU>(a, s); }
+void launch_mlp_proj_rows(const GemvArgs& a, hipStream_t s) { launch_rows<kMLP, 64, 8, PRO_PLAIN, EPI_RES>(a, s); }
 
 // Resident kernels of one device take turns: two at once could each hold CUs
 // that the other waits for.  While a turn lasts, its stream's work is enqueued
@@ -1034,21 +1170,24 @@ struct GptDecoder::Impl {
   uint32_t* hist = nullptr;     // the repetition-history prefix [kMaxHistory]
   TokenMail* mail = nullptr;    // the resident step kernel's words
   uint32_t epoch = 1;           // first tag epoch no launch has used
-  float* part = nullptr;        // attention splits: [20 heads][nsplit_max][66]
+  float* part = nullptr;        // attention splits: [8 query rows][20 heads][nsplit_max][66]
   int nsplit_max = 0;
 
   // check_stop: the launch does nothing once the stop token was predicted
   // (decode steps; the timing hook passes 0).
-  void launch_attention(const float* qv, const float* K, const float* V, float* out, int check_stop = 1) {
-    hipLaunchKernelGGL(attn_split_kernel, dim3(kHeads, nsplit_max), dim3(kAttnThreads), 0, s, qv, K, V, st, part, out,
-                       nsplit_max, check_stop);
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(kHeads), dim3(kHD), 0, s, st, part, out, nsplit_max, check_stop);
+  void launch_attention(const float* qv, const float* K, const float* V, float* out, int rows_z,
+                        int check_stop = 1) {
+    hipLaunchKernelGGL(attn_split_kernel, dim3(kHeads, nsplit_max, rows_z), dim3(kAttnThreads), 0, s, qv, K, V, st,
+                       part, out, nsplit_max, check_stop);
+    hipLaunchKernelGGL(attn_combine_kernel, dim3(kHeads, 1, rows_z), dim3(kHD), 0, s, st, part, out, nsplit_max,
+                       check_stop);
   }
   int* blk_idx;
   GptState* host_state = nullptr;  // pinned
   // row, row + head, token + head, kStepsPerCheck token steps, then the
-  // sampled forms of the last two; the same tokens by the resident kernel
-  hipGraphExec_t graph[10] = {};
+  // sampled forms of the last two; the same tokens by the resident kernel;
+  // a plain prefill chunk
+  hipGraphExec_t graph[11] = {};
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   // The resident step kernel decodes tokens (else the separate launches do):
   // all its workgroups fit the device, and no wait of it has run out.
@@ -1169,7 +1308,7 @@ struct GptDecoder::Impl {
                    align256(kVocab * f) + 2 * align256(kW * f) + align256((size_t)head_blocks() * f) +
                    align256((size_t)head_blocks() * 4) +
                    3 * align256((size_t)chunk_cap * kW * f) + align256((size_t)chunk_cap * kMLP * f) +
-                   align256((size_t)kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
+                   align256((size_t)kPlainRows * kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
                    align256((size_t)GptDecoder::kMaxHistory * 4) + align256(sizeof(TokenMail));
     ws.reserve(bytes);
@@ -1195,7 +1334,7 @@ struct GptDecoder::Impl {
     mail = static_cast<TokenMail*>(ws.take(sizeof(TokenMail)));
     GPT_OK(hipMemsetAsync(mail, 0, sizeof(TokenMail), s));  // no word carries a tag yet
     epoch = 1;
-    part = static_cast<float*>(ws.take((size_t)kHeads * nsplit_max * kPartF * f));
+    part = static_cast<float*>(ws.take((size_t)kPlainRows * kHeads * nsplit_max * kPartF * f));
     kc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
     vc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
     rows = static_cast<float*>(ws.take((size_t)rows_cap * kW * f));
@@ -1220,7 +1359,7 @@ struct GptDecoder::Impl {
       a.w = w.attn_w; a.bias = w.attn_b; a.N = kQKV; a.x = x; a.g1 = w.ln1_w; a.b1 = w.ln1_b;
       a.q = q; a.kc = K; a.vc = V;
       launch_qkv(a, s);
-      launch_attention(q, K, V, att);
+      launch_attention(q, K, V, att, 1);
       a = base_args();
       a.w = w.proj_w; a.bias = w.proj_b; a.N = kW; a.x = att; a.y = x;
       launch_attn_proj(a, s);
@@ -1311,11 +1450,44 @@ struct GptDecoder::Impl {
     }
   }
 
+  // One chunk of the plain prefill: up to kPlainRows prefix rows through every
+  // layer, fp32 throughout, each row with the decode step's bits.  (The products'
+  // split operands are not in use then; their buffers hold the fp32 rows.)
+  void enqueue_chunk() {
+    float *attr = reinterpret_cast<float*>(a16), *fcr = reinterpret_cast<float*>(fc16);
+    hipLaunchKernelGGL(embed_rows_kernel, dim3(1), dim3(256), 0, s, st, rows, xr);
+    for (int l = 0; l < L; ++l) {
+      const GptLayerDev& w = layer[l];
+      float* K = kc + (size_t)l * cap * kW;
+      float* V = vc + (size_t)l * cap * kW;
+      GemvArgs a = base_args();
+      a.w = w.attn_w; a.bias = w.attn_b; a.N = kQKV; a.x = xr; a.g1 = w.ln1_w; a.b1 = w.ln1_b;
+      a.q = qr; a.kc = K; a.vc = V;
+      launch_qkv_rows(a, s);
+      launch_attention(qr, K, V, attr, kPlainRows);
+      a = base_args();
+      a.w = w.proj_w; a.bias = w.proj_b; a.N = kW; a.x = attr; a.y = xr;
+      launch_attn_proj_rows(a, s);
+      a = base_args();
+      a.w = w.fc_w; a.bias = w.fc_b; a.N = kMLP; a.x = xr; a.g1 = w.ln2_w; a.b1 = w.ln2_b; a.y = fcr;
+      launch_fc_rows(a, s);
+      a = base_args();
+      a.w = w.mp_w; a.bias = w.mp_b; a.N = kW; a.x = fcr; a.y = xr;
+      launch_mlp_proj_rows(a, s);
+    }
+    hipLaunchKernelGGL(advance_rows_kernel, dim3(1), dim3(1), 0, s, st);
+    GPT_OK(hipGetLastError());
+  }
+
   // 0 row, 1 row + head, 2 token + head, 3 = 2 x kStepsPerCheck,
   // 4 token + head + sampler, 5 = 4 x kStepsPerCheck; 6 .. 9: 2 .. 5 by the
-  // resident kernel
+  // resident kernel; 10 plain prefill chunk
   void run_step(int which) {
     auto enqueue = [&] {
+      if (which == 10) {
+        enqueue_chunk();
+        return;
+      }
       if (which < 2) {
         enqueue_step(0, which == 1);
         return;
@@ -1352,14 +1524,9 @@ struct GptDecoder::Impl {
     GPT_OK(hipGraphLaunch(graph[which], s));
   }
 
-  // Prefix rows into the caches, in chunks of up to kPrefillRows rows, or one
-  // at a time through the decode step's kernels (`by_rows`: all fp32, whatever
-  // the values' range).  Returns the last row's hidden state (by_rows: NULL).
-  const float* prefill(int n, bool by_rows) {
-    if (by_rows) {
-      for (int i = 0; i < n; ++i) run_step(0);
-      return nullptr;
-    }
+  // Prefix rows into the caches: as row products in chunks of up to
+  // kPrefillRows rows (returns the last row's hidden state) ...
+  const float* prefill(int n) {
     const float* last = nullptr;
     for (int i = 0; i < n; i += chunk_cap) {
       const int M = std::min(chunk_cap, n - i);
@@ -1368,15 +1535,24 @@ struct GptDecoder::Impl {
     }
     return last;
   }
-  // env MIT2CFM_GPT_ROW_PREFILL=1: prefill one row at a time (for checking).
+  // ... or plain, fp32 whatever the values' range, in chunks of kPlainRows (213
+  // rows and one more 40.6 ms; one row at a time 140).
+  void prefill_plain(int n) {
+    if (row_prefill())
+      for (int i = 0; i < n; ++i) run_step(0);
+    else
+      for (int i = 0; i < n; i += kPlainRows) run_step(10);
+  }
+  // env MIT2CFM_GPT_ROW_PREFILL=1: plain, the prefix one row at a time (for checking).
   static bool row_prefill() {
     const char* e = std::getenv("MIT2CFM_GPT_ROW_PREFILL");
     return e && std::atoi(e) != 0;
   }
 
-  // kv: rows the caches hold once the prefill has run (0: rows join one by one)
+  // pend: prefix rows of the plain prefill; kv: rows the caches hold once the
+  // prefill has run (0: they join as the plain prefill goes)
   // steps: an upper bound of the steps that follow
-  void reset_state(int prefix_rows, int kv, bool hf, int steps, const GptDecoder::Sampling* smp = nullptr) {
+  void reset_state(int prefix_rows, int pend, int kv, bool hf, int steps, const GptDecoder::Sampling* smp = nullptr) {
     GptState h{};
     h.epoch = epoch;
     epoch += (uint32_t)steps;
@@ -1404,6 +1580,7 @@ struct GptDecoder::Impl {
     h.max_pred = pred_cap;
     h.cap = cap;
     h.rows = std::max(prefix_rows, 1);
+    h.pend = pend;
     *host_state = h;
     const uint32_t start = (uint32_t)kStart;
     GPT_OK(hipMemcpyAsync(st, host_state, sizeof(GptState), hipMemcpyHostToDevice, s));
@@ -1558,9 +1735,12 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   if (prefix_tokens > 0)
     GPT_OK(hipMemcpyAsync(d.rows, prefix, (size_t)prefix_tokens * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
   auto decode = [&](bool plain) {
-    d.reset_state(prefix_tokens, plain ? 0 : prefix_tokens, hf, steps, sampling);
+    d.reset_state(prefix_tokens, prefix_tokens, plain ? 0 : prefix_tokens, hf, steps, sampling);
     GPT_OK(hipEventRecord(d.ev[0], d.s));
-    d.prefill(prefix_tokens, plain);
+    if (plain)
+      d.prefill_plain(prefix_tokens);
+    else
+      d.prefill(prefix_tokens);
     GPT_OK(hipEventRecord(d.ev[1], d.s));
     int done = 0;
     while (done < steps) {
@@ -1586,7 +1766,7 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
     return d.host_state->overflow == 0 && d.host_state->aborted == 0;
   };
   // A call whose activations leave f16's range runs again the plain way, fp32
-  // throughout: rows prefilled one by one, tokens by the separate launches.
+  // throughout: rows prefilled in plain chunks, tokens by the separate launches.
   // One whose resident kernel had to give up (its workgroups could not all
   // run: another process keeps some of the GPU's CUs) runs again with those
   // launches, as do all that follow in this context.
@@ -1623,13 +1803,13 @@ uint32_t GptDecoder::cached_decode(const float* rows, int prefix_tokens, float* 
   if (!rows) throw std::invalid_argument("gpt: rows must not be NULL");
   d.ensure(prefix_tokens + 1, prefix_tokens + 1, 1);
   GPT_OK(hipMemcpyAsync(d.rows, rows, ((size_t)prefix_tokens + 1) * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
-  auto decode = [&](bool by_rows) {
-    d.reset_state(prefix_tokens + 1, 0, false, 1);
-    if (by_rows) {
-      d.prefill(prefix_tokens, true);
+  auto decode = [&](bool plain) {
+    d.reset_state(prefix_tokens + 1, prefix_tokens, 0, false, 1);
+    if (plain) {
+      d.prefill_plain(prefix_tokens);
       d.run_step(1);
     } else {  // the last row is known too: it goes through the layers with the others
-      d.enqueue_head(d.prefill(prefix_tokens + 1, false), false);
+      d.enqueue_head(d.prefill(prefix_tokens + 1), false);
       GPT_OK(hipGetLastError());
     }
     GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
@@ -1668,7 +1848,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
   }
   // A state with kKeys - 1 cached rows; the caches hold whatever they hold
   // (timing only).
-  d.reset_state(1, 0, false, 1);
+  d.reset_state(1, 0, 0, false, 1);
   d.host_state->kv = kKeys - 1;
   GPT_OK(hipMemcpyAsync(d.st, d.host_state, sizeof(GptState), hipMemcpyHostToDevice, d.s));
   GPT_OK(hipMemsetAsync(d.x, 0, kW * sizeof(float), d.s));
@@ -1722,7 +1902,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
         break;
       default:
         d.launch_attention(d.q, d.kc + (size_t)(i % d.L) * d.cap * kW, d.vc + (size_t)(i % d.L) * d.cap * kW,
-                           d.att, 0);
+                           d.att, 1, 0);
         break;
     }
   }

@@ -38,7 +38,8 @@ struct GptState {
                       //   empty one), 0: with the start token
   uint32_t epoch;     // tag epoch of step 0 (gpt_token.hip): step s uses epoch + s
   int32_t aborted;    // 1: a wait of the resident step kernel ran out
-  int32_t pad[9];
+  int32_t pend;       // prefix rows the plain prefill's chunks cover (rows 0..pend-1)
+  int32_t pad[8];
 };
 static_assert(sizeof(GptState) == 128, "GptState layout");
 
