@@ -489,6 +489,22 @@ mit2cfm_status mit2cfm_gpt_kv_sample(mit2cfm_ctx* ctx, const float* prefix, uint
 mit2cfm_status mit2cfm_gpt_cached_decode(mit2cfm_ctx* ctx, const float* rows, uint32_t prefix_tokens,
                                          float* ln_f, float* final_norm, float* logits, uint32_t* argmax);
 
+/* How the GPT calls of a context ran, counted since it was created.  Tokens
+ * are decoded by one resident kernel a step and a prefix goes through the
+ * layers as row products, both with f16 operand pairs; the plain forms, fp32
+ * throughout, take over where a value does not fit such a pair and where the
+ * resident kernel cannot have the GPU (its results are the same to fp32
+ * rounding). */
+typedef struct mit2cfm_gpt_counts {
+  uint64_t resident_steps; /* token steps by the resident kernel */
+  uint64_t plain_steps;    /* token steps by plain launches */
+  uint64_t row_prefills;   /* prefixes taken as row products */
+  uint64_t plain_prefills; /* prefixes taken by plain launches */
+  uint64_t range_reruns;   /* times a value did not fit and plain launches took over */
+  uint64_t wait_reruns;    /* times a wait of the resident kernel ran out and they did */
+} mit2cfm_gpt_counts;
+mit2cfm_status mit2cfm_gpt_get_counts(mit2cfm_ctx* ctx, mit2cfm_gpt_counts* counts);
+
 /* Measurement hook of the GPT decode step: enqueues `count` launches of one of
  * its kernels (cycling the layers' weights) on the context's stream without
  * waiting, for timing with events on mit2cfm_stream; count 0 launches

@@ -779,6 +779,16 @@ mit2cfm_status mit2cfm_gpt_layers(mit2cfm_ctx* ctx, uint32_t* layers) {
   });
 }
 
+mit2cfm_status mit2cfm_gpt_get_counts(mit2cfm_ctx* ctx, mit2cfm_gpt_counts* counts) {
+  if (!ctx) return fail(nullptr, MIT2CFM_E_ARG, "ctx must not be NULL");
+  return guarded(ctx, [&] {
+    require(counts != nullptr, "counts must not be NULL");
+    const mit2hip::GptDecoder::Counts c = ctx->eng->gpt().counts();
+    *counts = {c.resident_steps, c.plain_steps,  c.row_prefills,
+               c.plain_prefills, c.range_reruns, c.wait_reruns};
+  });
+}
+
 mit2cfm_status mit2cfm_gpt_kv_greedy(mit2cfm_ctx* ctx, const float* prefix, uint32_t prefix_tokens,
                                      uint32_t steps, int32_t hf_generate_positions,
                                      uint32_t* predicted_tokens, uint32_t* n_predicted,

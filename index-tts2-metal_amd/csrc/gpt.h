@@ -89,7 +89,14 @@ class GptDecoder {
   uint32_t cached_decode(const float* rows, int prefix_tokens, float* ln_f, float* final_norm,
                          float* logits);
 
-  // Launches one of the decode step's kernels `launches` times on the stream
+  // How the calls so far ran (mit2cfm_gpt_counts).
+  struct Counts {
+    uint64_t resident_steps = 0, plain_steps = 0, row_prefills = 0, plain_prefills = 0;
+    uint64_t range_reruns = 0, wait_reruns = 0;
+  };
+  const Counts& counts() const;
+
+  // Launches one of the plain decode step's kernels `launches` times on the stream
   // (for timing): 0 = c_attn (3840 x 1280), 1 = attn c_proj (1280 x 1280),
   // 2 = c_fc (5120 x 1280), 3 = mlp c_proj (1280 x 5120), 4 = mel_head
   // (8194 x 1280), 5 = cached attention at 1024 keys.  Returns the kernel's

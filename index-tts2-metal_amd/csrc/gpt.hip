@@ -1189,6 +1189,7 @@ struct GptDecoder::Impl {
   // a plain prefill chunk
   hipGraphExec_t graph[11] = {};
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+  GptDecoder::Counts counts;
   // The resident step kernel decodes tokens (else the separate launches do):
   // all its workgroups fit the device, and no wait of it has run out.
   bool resident = false;
@@ -1527,6 +1528,7 @@ struct GptDecoder::Impl {
   // Prefix rows into the caches: as row products in chunks of up to
   // kPrefillRows rows (returns the last row's hidden state) ...
   const float* prefill(int n) {
+    counts.row_prefills += n > 0;
     const float* last = nullptr;
     for (int i = 0; i < n; i += chunk_cap) {
       const int M = std::min(chunk_cap, n - i);
@@ -1538,6 +1540,7 @@ struct GptDecoder::Impl {
   // ... or plain, fp32 whatever the values' range, in chunks of kPlainRows (213
   // rows and one more 40.6 ms; one row at a time 140).
   void prefill_plain(int n) {
+    counts.plain_prefills += n > 0;
     if (row_prefill())
       for (int i = 0; i < n; ++i) run_step(0);
     else
@@ -1701,6 +1704,7 @@ GptDecoder::~GptDecoder() { delete d_; }
 
 size_t GptDecoder::weight_bytes() const { return d_->wa.used(); }
 int GptDecoder::layers() const { return d_->L; }
+const GptDecoder::Counts& GptDecoder::counts() const { return d_->counts; }
 
 void GptDecoder::kv_greedy(const float* prefix, int prefix_tokens, int steps, bool hf, Greedy& out) {
   generate(prefix, prefix_tokens, steps, hf, nullptr, out);
@@ -1758,6 +1762,7 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
       done += n;
       GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
       GPT_OK(hipStreamSynchronize(d.s));
+      (resident ? d.counts.resident_steps : d.counts.plain_steps) += (uint64_t)n;
       if (d.host_state->stopped || d.host_state->overflow || d.host_state->aborted) break;
     }
     GPT_OK(hipEventRecord(d.ev[2], d.s));
@@ -1772,10 +1777,13 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   // launches, as do all that follow in this context.
   bool plain = d.row_prefill();
   while (!decode(plain)) {
-    if (d.host_state->aborted)
+    if (d.host_state->aborted) {
+      d.counts.wait_reruns += 1;
       d.resident = false;
-    else
+    } else {
+      d.counts.range_reruns += 1;
       plain = true;
+    }
   }
   const GptState h = *d.host_state;
   out.first_stop_step = h.stop_step;
@@ -1816,7 +1824,12 @@ uint32_t GptDecoder::cached_decode(const float* rows, int prefix_tokens, float* 
     GPT_OK(hipStreamSynchronize(d.s));
     return d.host_state->overflow == 0;
   };
-  if (d.row_prefill() || !decode(false)) decode(true);
+  if (d.row_prefill()) {
+    decode(true);
+  } else if (!decode(false)) {
+    d.counts.range_reruns += 1;
+    decode(true);
+  }
   if (ln_f) GPT_OK(hipMemcpy(ln_f, d.lnf, kW * sizeof(float), hipMemcpyDeviceToHost));
   if (final_norm) GPT_OK(hipMemcpy(final_norm, d.fn, kW * sizeof(float), hipMemcpyDeviceToHost));
   if (logits) GPT_OK(hipMemcpy(logits, d.logits, kVocab * sizeof(float), hipMemcpyDeviceToHost));

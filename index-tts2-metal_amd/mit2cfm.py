@@ -123,6 +123,7 @@ def lib() -> ctypes.CDLL:
         "mit2cfm_write_image": (st, [vp, ctypes.c_char_p]),
         "mit2cfm_create_from_image": (st, [ctypes.c_char_p, i32, ctypes.POINTER(vp)]),
         "mit2cfm_gpt_layers": (st, [vp, _u32p]),
+        "mit2cfm_gpt_get_counts": (st, [vp, ctypes.POINTER(_GptCounts)]),
         "mit2cfm_gpt_kv_greedy": (st, [vp, _f32p, u32, u32, i32, _u32p, _u32p, _u32p, _u32p,
                                        ctypes.POINTER(i32), _f32p, ctypes.POINTER(ctypes.c_double)]),
         "mit2cfm_gpt_cached_decode": (st, [vp, _f32p, u32, _f32p, _f32p, _f32p, _u32p]),
@@ -138,6 +139,11 @@ def lib() -> ctypes.CDLL:
         fn.argtypes = args
     _lib = L
     return L
+
+
+class _GptCounts(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_uint64) for n in ("resident_steps", "plain_steps", "row_prefills", "plain_prefills",
+                                               "range_reruns", "wait_reruns")]
 
 
 class _GptSampling(ctypes.Structure):
@@ -640,6 +646,12 @@ class Context:
         n = np.zeros(1, np.uint32)
         self._c(lib().mit2cfm_gpt_layers(self._h, _pu(n)))
         return int(n[0])
+
+    def gpt_counts(self) -> dict:
+        """How the GPT calls of this context ran so far (mit2cfm_gpt_counts)."""
+        c = _GptCounts()
+        self._c(lib().mit2cfm_gpt_get_counts(self._h, ctypes.byref(c)))
+        return {n: int(getattr(c, n)) for n, _ in c._fields_}
 
     def gpt_kv_greedy(self, prefix, steps: int, hf_generate_positions: bool = False) -> dict:
         """run_gpt_kv_greedy (gpt.cpp:1877): prefix [P, 1280] -> dict with

@@ -35,6 +35,13 @@ def _ensure_built():
         __graft_entry__.build()
 
 
+def gpt_paths(ctx, call):
+    """A GPT call's result, and how it ran: the counts it added (zeros left out)."""
+    before = ctx.gpt_counts()
+    out = call()
+    return out, {k: n - before[k] for k, n in ctx.gpt_counts().items() if n != before[k]}
+
+
 @pytest.fixture(scope="session")
 def mit2():
     _ensure_built()

@@ -19,6 +19,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from conftest import gpt_paths
+
 pytestmark = pytest.mark.gpu
 
 W = 1280
@@ -40,11 +42,16 @@ def _rows(n, seed):
     return (np.random.default_rng(seed).standard_normal((n, W)) * 0.05).astype(np.float32)
 
 
-def _both(ctx, rows, monkeypatch):
+def _both(ctx, rows, monkeypatch, fits=True):
+    """The call as row products and plain; `fits`: its values fit f16, so the
+    first must not have fallen back to the second (else it must have)."""
+    plain = {"plain_prefills": 1} if len(rows) > 1 else {}
     monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
-    got = ctx.gpt_cached_decode(rows, len(rows) - 1)
+    got, how = gpt_paths(ctx, lambda: ctx.gpt_cached_decode(rows, len(rows) - 1))
+    assert how == ({"row_prefills": 1} if fits else {"row_prefills": 1, "range_reruns": 1, **plain})
     monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
-    ref = ctx.gpt_cached_decode(rows, len(rows) - 1)
+    ref, how = gpt_paths(ctx, lambda: ctx.gpt_cached_decode(rows, len(rows) - 1))
+    assert how == plain
     return got, ref
 
 
@@ -77,7 +84,9 @@ def test_a_row_does_not_depend_on_the_prefix_length(mit2, tensors):
         ref = None
         for M in (1, 2, 16, 33, 64, 65, 128, 129, 193, 213, 257, 385, 450, 833, 1024, 1025, 1100):
             print(f"row bits M={M}", flush=True)
-            got = c.gpt_cached_decode(np.concatenate([np.repeat(-x, M - 1, 0), x]), M - 1)
+            rows = np.concatenate([np.repeat(-x, M - 1, 0), x])
+            got, how = gpt_paths(c, lambda: c.gpt_cached_decode(rows, M - 1))
+            assert how == {"row_prefills": 1}
             ref = got if ref is None else ref
             for a, r in zip(got[:3], ref[:3]):
                 assert np.isfinite(a).all() and np.array_equal(a, r)
@@ -89,7 +98,8 @@ def test_prefill_caches_serve_the_decode(ctx2, monkeypatch):
     """Tokens decoded after the prefill read the caches it wrote."""
     prefix = _rows(97, 5)
     monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
-    got = ctx2.gpt_kv_greedy(prefix, 20)
+    got, how = gpt_paths(ctx2, lambda: ctx2.gpt_kv_greedy(prefix, 20))
+    assert how == {"row_prefills": 1, "resident_steps": 20}
     monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
     ref = ctx2.gpt_kv_greedy(prefix, 20)
     assert got["predicted"].tolist() == ref["predicted"].tolist()
@@ -116,12 +126,13 @@ def test_values_past_f16_take_the_row_prefill(mit2, tensors, gpt2_t, monkeypatch
         t["gpt.gpt.h.0.attn.c_attn.bias"] = b
     c = mit2.Context({**tensors, **t}, device=0)
     try:
-        got, ref = _both(c, _rows(21, 9), monkeypatch)
+        got, ref = _both(c, _rows(21, 9), monkeypatch, fits=False)
         for a, b in zip(got[:3], ref[:3]):
             assert np.isfinite(a).all() and np.array_equal(a, b)
         assert got[3] == ref[3]
         monkeypatch.delenv("MIT2CFM_GPT_ROW_PREFILL", raising=False)
-        g = c.gpt_kv_greedy(_rows(21, 9), 12)
+        g, how = gpt_paths(c, lambda: c.gpt_kv_greedy(_rows(21, 9), 12))
+        assert how["range_reruns"] == 1 and how["plain_prefills"] == 1 and how["plain_steps"] == 12
         monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
         r = c.gpt_kv_greedy(_rows(21, 9), 12)
         assert g["predicted"].tolist() == r["predicted"].tolist()

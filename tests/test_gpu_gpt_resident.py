@@ -18,6 +18,8 @@ import threading
 import numpy as np
 import pytest
 
+from conftest import gpt_paths
+
 pytestmark = pytest.mark.gpu
 
 W = 1280
@@ -54,6 +56,16 @@ def _rows(n, seed):
     return (np.random.default_rng(seed).standard_normal((n, W)) * 0.05).astype(np.float32)
 
 
+def _pair(a, b, steps, P, call):
+    """`call` on the resident context and on the plain one, each on its own path."""
+    prefill = {"row_prefills": 1} if P else {}
+    ra, how = gpt_paths(a, lambda: call(a))
+    assert how == {"resident_steps": steps, **prefill}
+    rb, how = gpt_paths(b, lambda: call(b))
+    assert how == {"plain_steps": steps, **prefill}
+    return ra, rb
+
+
 def _same(a, b):
     assert a["predicted"].tolist() == b["predicted"].tolist()
     assert a["input_tokens"].tolist() == b["input_tokens"].tolist()
@@ -66,7 +78,7 @@ def _same(a, b):
 def test_greedy_equals_separate_launches(pair2, P, steps):
     print(f"resident greedy P={P} steps={steps}", flush=True)
     x = _rows(P, P)
-    _same(pair2[0].gpt_kv_greedy(x, steps, True), pair2[1].gpt_kv_greedy(x, steps, True))
+    _same(*_pair(*pair2, steps, P, lambda c: c.gpt_kv_greedy(x, steps, True)))
 
 
 @pytest.mark.parametrize("layers", [1, 3])
@@ -75,7 +87,7 @@ def test_layer_counts(mit2, tensors, monkeypatch, layers):
     a, b = mit2.Context(t, device=0), _plain(mit2, t, monkeypatch)
     try:
         print(f"resident greedy layers={layers}", flush=True)
-        _same(a.gpt_kv_greedy(_rows(7, 1), 9), b.gpt_kv_greedy(_rows(7, 1), 9))
+        _same(*_pair(a, b, 9, 7, lambda c: c.gpt_kv_greedy(_rows(7, 1), 9)))
     finally:
         a.close()
         b.close()
@@ -83,8 +95,8 @@ def test_layer_counts(mit2, tensors, monkeypatch, layers):
 
 def test_sampled_equals_separate_launches(pair2):
     x = _rows(33, 2)
-    a, b = (c.gpt_kv_sample(x, 20, 11, hf_generate_positions=True, history=[1] * 33 + [8192], **SAMPLING) for c in pair2)
-    _same(a, b)
+    _same(*_pair(*pair2, 20, 33, lambda c: c.gpt_kv_sample(x, 20, 11, hf_generate_positions=True,
+                                                           history=[1] * 33 + [8192], **SAMPLING)))
 
 
 def test_repeats_to_the_bit(pair2):
@@ -92,7 +104,8 @@ def test_repeats_to_the_bit(pair2):
     x = _rows(40, 3)
     a = pair2[0].gpt_kv_greedy(x, 30)
     for _ in range(5):
-        b = pair2[0].gpt_kv_greedy(x, 30)
+        b, how = gpt_paths(pair2[0], lambda: pair2[0].gpt_kv_greedy(x, 30))
+        assert how == {"row_prefills": 1, "resident_steps": 30}
         assert a["predicted"].tolist() == b["predicted"].tolist()
         assert np.array_equal(a["last_logits"], b["last_logits"])
 
@@ -120,6 +133,8 @@ def test_contexts_on_threads_take_turns(mit2, tensors):
             for g in got[i]:
                 assert g["predicted"].tolist() == want[i]["predicted"].tolist()
                 assert np.array_equal(g["last_logits"], want[i]["last_logits"])
+            n = ctx[i].gpt_counts()
+            assert n["resident_steps"] == 5 * 60 and n["plain_steps"] == n["wait_reruns"] == n["range_reruns"] == 0
     finally:
         for c in ctx:
             c.close()
@@ -134,7 +149,9 @@ def test_a_wait_that_runs_out_falls_back(mit2, tensors, monkeypatch):
     a = mit2.Context(t, device=0)
     try:
         x = _rows(25, 4)
-        ra, rb = a.gpt_kv_greedy(x, 12), b.gpt_kv_greedy(x, 12)
+        ra, how = gpt_paths(a, lambda: a.gpt_kv_greedy(x, 12))
+        assert how["wait_reruns"] == 1 and how["plain_steps"] == 12 and "range_reruns" not in how
+        rb = b.gpt_kv_greedy(x, 12)
         assert ra["predicted"].tolist() == rb["predicted"].tolist()
         assert np.array_equal(ra["last_logits"], rb["last_logits"])
         ra = a.gpt_kv_sample(x, 12, 5, **SAMPLING)
@@ -159,7 +176,9 @@ def test_decode_values_past_f16(mit2, tensors, monkeypatch, where):
     a, b = mit2.Context(t, device=0), _plain(mit2, t, monkeypatch)
     try:
         for _ in range(2):
-            ra, rb = a.gpt_kv_greedy(_rows(0, 0), 10), b.gpt_kv_greedy(_rows(0, 0), 10)
+            ra, how = gpt_paths(a, lambda: a.gpt_kv_greedy(_rows(0, 0), 10))
+            assert how["range_reruns"] == 1 and how["plain_steps"] == 10 and "wait_reruns" not in how
+            rb = b.gpt_kv_greedy(_rows(0, 0), 10)
             assert ra["predicted"].tolist() == rb["predicted"].tolist()
             assert np.isfinite(ra["last_logits"]).all()
             assert np.array_equal(ra["last_logits"], rb["last_logits"])
