@@ -439,6 +439,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
                                                                 uint32_t* predicted, uint32_t* inputs,
                                                                 float* proc, const uint32_t* hist_prefix) {
   if (st->stopped) return;
+  if (st->failed()) {  // the host takes the step again
+    if (threadIdx.x == 0) st->stopped = 1;
+    return;
+  }
   __shared__ float sv[kSortN];
   __shared__ uint32_t si[kSortN];
   __shared__ uint32_t seen[(kVocab + 31) / 32];
@@ -831,6 +835,10 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* blk_val, cons
                                                       GptState* st, uint32_t* predicted, uint32_t* inputs,
                                                       int check_stop) {
   if (check_stop && st->stopped) return;
+  if (check_stop && st->failed()) {  // the host takes the step again
+    if (threadIdx.x == 0) st->stopped = 1;
+    return;
+  }
   __shared__ float wv[16];
   __shared__ int wi[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1738,54 +1746,62 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   d.ensure(prefix_tokens + steps + 1, prefix_tokens + 1, steps);
   if (prefix_tokens > 0)
     GPT_OK(hipMemcpyAsync(d.rows, prefix, (size_t)prefix_tokens * kW * sizeof(float), hipMemcpyHostToDevice, d.s));
-  auto decode = [&](bool plain) {
+  // Rows and tokens go through the row products and the resident kernel, or
+  // plain.  A step that fails (a value past f16's range, a wait of the resident
+  // kernel that ran out) picks no token and stops the steps behind it, so the
+  // decode goes on from that step with the plain launches.  A prefix whose
+  // values do not fit is prefilled again, plain, and all its tokens are plain.
+  bool plain = d.row_prefill();
+  GptState& h = *d.host_state;
+  bool begun = false;
+  auto prefill = [&] {
     d.reset_state(prefix_tokens, prefix_tokens, plain ? 0 : prefix_tokens, hf, steps, sampling);
-    GPT_OK(hipEventRecord(d.ev[0], d.s));
+    if (!begun) GPT_OK(hipEventRecord(d.ev[0], d.s));  // (a second prefill counts as part of the first)
+    begun = true;
     if (plain)
       d.prefill_plain(prefix_tokens);
     else
       d.prefill(prefix_tokens);
     GPT_OK(hipEventRecord(d.ev[1], d.s));
-    int done = 0;
-    while (done < steps) {
-      const int n = std::min(kStepsPerCheck, steps - done);
-      const bool resident = d.resident && !plain;
-      const int token = (sampling ? 4 : 2) + (resident ? 4 : 0);
-      {
-        std::unique_ptr<ResidentTurn> turn(resident ? new ResidentTurn(d.s) : nullptr);
-        if (n == kStepsPerCheck) {
-          d.run_step(token + 1);  // one graph of kStepsPerCheck steps
-        } else {
-          for (int i = 0; i < n; ++i) d.run_step(token);
-        }
-      }
-      done += n;
-      GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
-      GPT_OK(hipStreamSynchronize(d.s));
-      (resident ? d.counts.resident_steps : d.counts.plain_steps) += (uint64_t)n;
-      if (d.host_state->stopped || d.host_state->overflow || d.host_state->aborted) break;
-    }
-    GPT_OK(hipEventRecord(d.ev[2], d.s));
-    GPT_OK(hipMemcpyAsync(d.host_state, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
-    GPT_OK(hipStreamSynchronize(d.s));
-    return d.host_state->overflow == 0 && d.host_state->aborted == 0;
   };
-  // A call whose activations leave f16's range runs again the plain way, fp32
-  // throughout: rows prefilled in plain chunks, tokens by the separate launches.
-  // One whose resident kernel had to give up (its workgroups could not all
-  // run: another process keeps some of the GPU's CUs) runs again with those
-  // launches, as do all that follow in this context.
-  bool plain = d.row_prefill();
-  while (!decode(plain)) {
-    if (d.host_state->aborted) {
-      d.counts.wait_reruns += 1;
-      d.resident = false;
-    } else {
+  prefill();
+  for (int done = 0;;) {
+    const bool resident = d.resident && !plain;
+    const int n = std::min(kStepsPerCheck, steps - done);
+    if (n > 0) {
+      std::unique_ptr<ResidentTurn> turn(resident ? new ResidentTurn(d.s) : nullptr);
+      const int token = (sampling ? 4 : 2) + (resident ? 4 : 0);
+      if (n == kStepsPerCheck) {
+        d.run_step(token + 1);  // one graph of kStepsPerCheck steps
+      } else {
+        for (int i = 0; i < n; ++i) d.run_step(token);
+      }
+    }
+    GPT_OK(hipMemcpyAsync(&h, d.st, sizeof(GptState), hipMemcpyDeviceToHost, d.s));
+    GPT_OK(hipStreamSynchronize(d.s));
+    (resident ? d.counts.resident_steps : d.counts.plain_steps) += (uint64_t)(h.step - done);
+    done = h.step;
+    if (h.overflow) {
       d.counts.range_reruns += 1;
       plain = true;
+      prefill();
+    } else if (h.failed()) {
+      if (h.aborted) {  // another process keeps some of the GPU's CUs
+        d.counts.wait_reruns += 1;
+        d.resident = false;
+      } else {
+        d.counts.range_reruns += 1;
+      }
+      plain = true;
+      h.unfit = h.aborted = h.stopped = 0;
+      h.kv = prefix_tokens + done;
+      GPT_OK(hipMemcpyAsync(d.st, &h, sizeof(GptState), hipMemcpyHostToDevice, d.s));
+    } else if (h.stopped || done >= steps) {
+      break;
     }
   }
-  const GptState h = *d.host_state;
+  GPT_OK(hipEventRecord(d.ev[2], d.s));
+  GPT_OK(hipStreamSynchronize(d.s));
   out.first_stop_step = h.stop_step;
   out.predicted.assign((size_t)h.n_pred, 0);
   out.input_tokens.assign((size_t)h.n_in, 0);

@@ -27,7 +27,7 @@ struct GptState {
   int32_t max_pred;   // capacity of the predicted array (inputs: + 1)
   int32_t cap;        // rows of each key/value cache
   int32_t rows;       // rows of the prefix buffer
-  int32_t overflow;   // 1: a prefill value did not fit a split f16 pair
+  int32_t overflow;   // 1: a value of the row-product prefill did not fit a split f16 pair
   int32_t top_k;      // sampling (sample_kernel): top-k (0: off)
   float temperature;  //   temperature, top-p, repetition penalty
   float top_p;
@@ -37,9 +37,13 @@ struct GptState {
   int32_t hist_given; //   1: the history starts with the caller's prefix (even an
                       //   empty one), 0: with the start token
   uint32_t epoch;     // tag epoch of step 0 (gpt_token.hip): step s uses epoch + s
+  int32_t unfit;      // 1: a value of the resident step kernel did not fit one
   int32_t aborted;    // 1: a wait of the resident step kernel ran out
   int32_t pend;       // prefix rows the plain prefill's chunks cover (rows 0..pend-1)
-  int32_t pad[8];
+  int32_t pad[7];
+
+  // The logits are worthless: no token is picked from them.
+  __host__ __device__ bool failed() const { return (overflow | unfit | aborted) != 0; }
 };
 static_assert(sizeof(GptState) == 128, "GptState layout");
 

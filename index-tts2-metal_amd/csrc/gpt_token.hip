@@ -239,7 +239,7 @@ __device__ __forceinline__ void put_split(half_t* hi, half_t* lo, int i, int ste
     *reinterpret_cast<half2v*>(hi + i + (e / 2) * step) = half2v{h0, h1};
     *reinterpret_cast<half2v*>(lo + i + (e / 2) * step) = half2v{l0, l1};
   }
-  if (nan || big > kSplitMax) st->overflow = 1;
+  if (nan || big > kSplitMax) st->unfit = 1;
 }
 
 template <typename T>
@@ -629,7 +629,7 @@ __device__ __forceinline__ void poll_waves(const TokenArgs& a, Lds& s, int wg, i
       s.x[0][pos(i / 2) + (i & 1)] = h;
       s.x[1][pos(i / 2) + (i & 1)] = l;
     }
-    if (!fits) a.st->overflow = 1;
+    if (!fits) a.st->unfit = 1;
   };
   for (int i = lane + 64 * pw; i < 3 * kR3W - kW; i += 64 * kPW) s.x[0][kW + i] = s.x[1][kW + i] = (half_t)0.f;
   for (int i = lane + 64 * pw; i < 3 * kR3F - kMLP; i += 64 * kPW) s.xf[0][kMLP + i] = s.xf[1][kMLP + i] = (half_t)0.f;
