@@ -1199,8 +1199,13 @@ struct GptDecoder::Impl {
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   GptDecoder::Counts counts;
   // The resident step kernel decodes tokens (else the separate launches do):
-  // all its workgroups fit the device, and no wait of it has run out.
+  // all its workgroups fit the device.  A call in which a wait of it ran out (a
+  // neighbour kept some of the CUs for about a second) leaves the next calls
+  // plain: 1, then 2, 4 .. kMostSkipped of them while that goes on, as each try
+  // costs the wait; 1 again after a call that ran through.
   bool resident = false;
+  static constexpr int kMostSkipped = 64;
+  int skip_calls = 0, next_skip = 1;
   uint32_t spin_limit = 1u << 20;  // env MIT2CFM_GPT_SPIN_LIMIT (for checking: 1 gives up at once)
   size_t layer_stride = 0;  // bytes from a layer's arrays to the next's
   bool use_graph = true;  // env MIT2CFM_GRAPH=0: launch every kernel directly (for profilers)
@@ -1752,6 +1757,11 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   // decode goes on from that step with the plain launches.  A prefix whose
   // values do not fit is prefilled again, plain, and all its tokens are plain.
   bool plain = d.row_prefill();
+  bool resident = d.resident && !plain;
+  if (resident && steps > 0 && d.skip_calls > 0) {
+    d.skip_calls -= 1;
+    resident = false;
+  }
   GptState& h = *d.host_state;
   bool begun = false;
   auto prefill = [&] {
@@ -1766,7 +1776,6 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
   };
   prefill();
   for (int done = 0;;) {
-    const bool resident = d.resident && !plain;
     const int n = std::min(kStepsPerCheck, steps - done);
     if (n > 0) {
       std::unique_ptr<ResidentTurn> turn(resident ? new ResidentTurn(d.s) : nullptr);
@@ -1784,19 +1793,22 @@ void GptDecoder::generate(const float* prefix, int prefix_tokens, int steps, boo
     if (h.overflow) {
       d.counts.range_reruns += 1;
       plain = true;
+      resident = false;
       prefill();
     } else if (h.failed()) {
-      if (h.aborted) {  // another process keeps some of the GPU's CUs
+      if (h.aborted) {
         d.counts.wait_reruns += 1;
-        d.resident = false;
+        d.skip_calls = d.next_skip;
+        d.next_skip = std::min(2 * d.next_skip, d.kMostSkipped);
       } else {
         d.counts.range_reruns += 1;
       }
-      plain = true;
+      resident = false;
       h.unfit = h.aborted = h.stopped = 0;
       h.kv = prefix_tokens + done;
       GPT_OK(hipMemcpyAsync(d.st, &h, sizeof(GptState), hipMemcpyHostToDevice, d.s));
     } else if (h.stopped || done >= steps) {
+      if (resident && done > 0) d.next_skip = 1;
       break;
     }
   }

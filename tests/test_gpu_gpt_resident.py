@@ -154,10 +154,13 @@ def test_a_wait_that_runs_out_falls_back(mit2, tensors, monkeypatch):
         rb = b.gpt_kv_greedy(x, 12)
         assert ra["predicted"].tolist() == rb["predicted"].tolist()
         assert np.array_equal(ra["last_logits"], rb["last_logits"])
-        ra = a.gpt_kv_sample(x, 12, 5, **SAMPLING)
+        # the resident kernel is tried again after 1, 2, 4 .. plain calls
         rb = b.gpt_kv_sample(x, 12, 5, **SAMPLING)
-        assert ra["predicted"].tolist() == rb["predicted"].tolist()
-        assert np.array_equal(ra["last_logits"], rb["last_logits"])
+        for gave_up in (0, 1, 0, 0, 1, 0, 0, 0, 0, 1, 0):
+            ra, how = gpt_paths(a, lambda: a.gpt_kv_sample(x, 12, 5, **SAMPLING))
+            assert how == {"row_prefills": 1, "plain_steps": 12, **({"wait_reruns": 1} if gave_up else {})}
+            assert ra["predicted"].tolist() == rb["predicted"].tolist()
+            assert np.array_equal(ra["last_logits"], rb["last_logits"])
     finally:
         a.close()
         b.close()
