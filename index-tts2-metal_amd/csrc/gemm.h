@@ -102,6 +102,7 @@ struct GemmArgs {
   int ldc32b = 0;
   float* C32c = nullptr;             // EPI_KVCACHE: the value cache
   int* overflow = nullptr;           // EPI_GELU16: set to 1 when an output does not fit f16
+  uint32_t* row_small = nullptr;     //   ... and the rows' counts (count_small)
   const float* cond = nullptr;       // EPI_GATE: [a(512) | b(512)] global conditioning
   const uint32_t* mask = nullptr;    // per-row 0/1 (WaveNet epilogues)
   const float* rp = nullptr;         // EPI_FINALSKIP: res_projection [M][512]
@@ -201,8 +202,21 @@ __device__ inline void split_f16(float v, half_t& hi, half_t& lo) {
   lo = (half_t)((v - (float)hi) * kSplitScale);
 }
 
-// Largest magnitude a split pair holds (its hi half is finite).
+// What a split pair holds: a magnitude up to kSplitMax (its hi half is finite),
+// to 2^-23 of itself from kSplitFull on and to 2^-36 below it (the lo half's
+// denormal step).  A row of a product's input whose largest value is at least
+// kSplitFull, or is 0, thus enters to 2^-23 of that value, as fp32 sums over the
+// row would round it anyway; one that is all smaller does not fit.
 constexpr float kSplitMax = 65504.0f;
+constexpr float kSplitFull = 1.0f / 8192.0f;
+// A row made by several waves, in `blocks` parts: each part without a value of
+// kSplitFull (rarely any) counts itself at *small, 0 before; the last of them all
+// reports the row when `some` part of it is not 0.
+__device__ __forceinline__ void count_small(uint32_t* small, uint32_t blocks, bool some, int* overflow) {
+  const uint32_t add = some ? 0x10001u : 1u;
+  const uint32_t n = atomicAdd(small, add) + add;
+  if ((n & 0xffffu) == blocks && (n >> 16) != 0) *overflow = 1;
+}
 
 // cpu_gelu_new (tokenizer_tests.cpp:3931-3945)
 __device__ __forceinline__ float gelu_new(float v) {

@@ -1027,6 +1027,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
 #pragma unroll
       for (int q = 0; q < (NI + 1) / 2; ++q) ssq[q] = s1[q] = 0.0f;
       float4 pv = make_float4(0.f, 0.f, 0.f, 0.f);  // column pairs: the even block's outputs
+      [[maybe_unused]] float fit_big = 0.f;         // EPI_GELU16: the largest magnitude
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
         const int n = colj(j);
@@ -1097,6 +1098,7 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
           if (!(fabsf(y.x) <= kSplitMax && fabsf(y.y) <= kSplitMax && fabsf(y.z) <= kSplitMax &&
                 fabsf(y.w) <= kSplitMax))
             *p.overflow = 1;
+          fit_big = fmaxf(fit_big, fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
           st16s(p.C16 + (size_t)m * p.ldc16 + n, y.x, y.y, y.z, y.w);
         } else if constexpr (EPI == EPI_KVCACHE) {
           if (n < kGptW) {
@@ -1135,6 +1137,15 @@ __global__ __launch_bounds__(64 * WM * WN * (PIPE ? 1 : KG)) void gemm_kernel(Ge
           *reinterpret_cast<float4*>(p.C32 + (size_t)m * p.ldc32 + n) =
               make_float4((o.x + v.x) * mk + r.x, (o.y + v.y) * mk + r.y, (o.z + v.z) * mk + r.z,
                           (o.w + v.w) * mk + r.w);
+        }
+      }
+      if constexpr (EPI == EPI_GELU16) {  // the four lanes of a row hold its part, WTN columns
+        auto rows = [](uint64_t b) { return (uint32_t)(b | b >> 16 | b >> 32 | b >> 48) & 0xffffu; };
+        const uint32_t small = rows(__ballot(live)) & ~rows(__ballot(fit_big >= kSplitFull));
+        if (small) {
+          const uint32_t some = rows(__ballot(fit_big > 0.f));
+          if (lane < 16 && (small >> lane & 1u))
+            count_small(p.row_small + m, (uint32_t)(p.N / WTN), some >> lane & 1u, p.overflow);
         }
       }
       if constexpr (EPI == EPI_F32) {
@@ -2108,7 +2119,7 @@ hipError_t launch_gemm_rows(const GemmArgs& a, EpiMode epi, hipStream_t stream) 
     return hipErrorInvalidValue;
   if (epi == EPI_KVCACHE && a.N == 3 * kGptW && a.C32 && a.C32b && a.C32c && a.T >= 0 && a.T + a.M <= a.Tpad)
     return launch_rows_epi<EPI_KVCACHE>(a, stream);
-  if (epi == EPI_GELU16 && a.C16 && a.c16_lo && a.overflow) return launch_rows_epi<EPI_GELU16>(a, stream);
+  if (epi == EPI_GELU16 && a.C16 && a.c16_lo && a.overflow && a.row_small) return launch_rows_epi<EPI_GELU16>(a, stream);
   if (epi == EPI_ROWS && a.C32 && a.res) return launch_rows_epi<EPI_ROWS>(a, stream);
   return hipErrorInvalidValue;
 }

@@ -26,10 +26,10 @@
 // weights once costs, the rest the latency of 24 x 7 dependent launches.
 //
 // A step normally runs as one resident kernel (gpt_token.hip); the kernels
-// below are its plain form, fp32 throughout, one launch a product: for values
-// past f16's range and for a GPU that cannot hold all of that kernel's
-// workgroups at once; past f16's range the prefix goes in chunks of 8 rows
-// through their multi-row form.
+// below are its plain form, fp32 throughout, one launch a product: for inputs
+// that f16 pairs do not hold (kSplitMax, kSplitFull) and for a GPU that cannot
+// hold all of that kernel's workgroups at once.  A prefix that pairs do not hold
+// goes through their multi-row form, 8 rows at a time.
 //
 // Every matrix-vector product reads its weights from HBM: each once per
 // step (f16, 0.98 GB for 24 layers) and used for one multiply-add.  The GEMV
@@ -1174,6 +1174,7 @@ struct GptDecoder::Impl {
   int chunk_cap = 0;            // rows of the prefill chunk buffers
   float *xr, *qr;               // a prefill chunk's rows: the residual stream and the queries
   half_t *a16, *fc16;           //   the products' split operands [2][rows][1280] and [2][rows][5120]
+  uint32_t* row_small = nullptr;  //   counts [layer][attention, gelu][rows] (count_small)
   float* proc = nullptr;        // the sampler's processed logits [8194]
   uint32_t* hist = nullptr;     // the repetition-history prefix [kMaxHistory]
   TokenMail* mail = nullptr;    // the resident step kernel's words
@@ -1324,7 +1325,8 @@ struct GptDecoder::Impl {
                    3 * align256((size_t)chunk_cap * kW * f) + align256((size_t)chunk_cap * kMLP * f) +
                    align256((size_t)kPlainRows * kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
-                   align256((size_t)GptDecoder::kMaxHistory * 4) + align256(sizeof(TokenMail));
+                   align256((size_t)GptDecoder::kMaxHistory * 4) + align256(sizeof(TokenMail)) +
+                   align256((size_t)2 * L * chunk_cap * 4);
     ws.reserve(bytes);
     st = static_cast<GptState*>(ws.take(sizeof(GptState)));
     predicted = static_cast<uint32_t*>(ws.take((size_t)pred_cap * 4));
@@ -1347,6 +1349,7 @@ struct GptDecoder::Impl {
     nsplit_max = cap / kChunk;
     mail = static_cast<TokenMail*>(ws.take(sizeof(TokenMail)));
     GPT_OK(hipMemsetAsync(mail, 0, sizeof(TokenMail), s));  // no word carries a tag yet
+    row_small = static_cast<uint32_t*>(ws.take((size_t)2 * L * chunk_cap * 4));
     epoch = 1;
     part = static_cast<float*>(ws.take((size_t)kPlainRows * kHeads * nsplit_max * kPartF * f));
     kc = static_cast<float*>(ws.take((size_t)L * cap * kW * f));
@@ -1429,7 +1432,7 @@ struct GptDecoder::Impl {
   // read once per chunk, so a prefix costs about one pass over the weights
   // and its arithmetic.  The activations are fp32 between the products and
   // enter each as a split f16 pair (fp32-level products: the weights are
-  // exact in f16); a value that does not fit one sets st->overflow.
+  // exact in f16); a row that does not fit them sets st->overflow.
   void enqueue_rows(int r0, int M) {
     const size_t lo = (size_t)chunk_cap * kW, fc_lo = (size_t)chunk_cap * kMLP;
     const float* xin = rows + (size_t)r0 * kW;  // the residual stream: the prefix rows, then xr
@@ -1441,12 +1444,13 @@ struct GptDecoder::Impl {
       const GptLayerDev& w = layer[l];
       float* K = kc + (size_t)l * cap * kW;
       float* V = vc + (size_t)l * cap * kW;
-      GPT_OK(launch_gpt_ln_rows(xin, w.ln1_w, w.ln1_b, M, a16, lo, ovf, s));
+      uint32_t* small = row_small + (size_t)2 * l * chunk_cap;
+      GPT_OK(launch_gpt_ln_rows(xin, w.ln1_w, w.ln1_b, M, a16, lo, ovf, s, row_small, l == 0 ? 2 * L : 0, chunk_cap));
       GemmArgs a = g;
       a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.attn_w; a.ldw = kW; a.N = kQKV; a.bias = w.attn_b;
       a.C32 = qr; a.ldc32 = kW; a.C32b = K; a.C32c = V; a.Tpad = cap; a.T = r0;
       GPT_OK(launch_gemm_rows(a, EPI_KVCACHE, s));
-      GPT_OK(launch_gpt_attn_rows(qr, K, V, cap, r0, M, a16, lo, ovf, s));
+      GPT_OK(launch_gpt_attn_rows(qr, K, V, cap, r0, M, a16, lo, ovf, small, s));
       a = g;
       a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.proj_w; a.ldw = kW; a.N = kW; a.bias = w.proj_b;
       a.res = xin; a.ldres = kW; a.C32 = xr; a.ldc32 = kW;
@@ -1456,6 +1460,7 @@ struct GptDecoder::Impl {
       a = g;
       a.A = a16; a.lda = kW; a.a_lo = lo; a.K = kW; a.W = w.fc_w; a.ldw = kW; a.N = kMLP; a.bias = w.fc_b;
       a.C16 = fc16; a.ldc16 = kMLP; a.c16_lo = fc_lo; a.overflow = ovf;
+      a.row_small = small + chunk_cap;
       GPT_OK(launch_gemm_rows(a, EPI_GELU16, s));
       a = g;
       a.A = fc16; a.lda = kMLP; a.a_lo = fc_lo; a.K = kMLP; a.W = w.mp_w; a.ldw = kMLP; a.N = kW; a.bias = w.mp_b;

@@ -12,8 +12,9 @@ namespace {
 
 constexpr int kHeads = 20, kHD = 64;
 
-// Four values as a split pair; reports one that does not fit (or is NaN).
-__device__ __forceinline__ void store_split4(half_t* dst, size_t lo, float4 v, int* overflow) {
+// Four values as a split pair; reports one that is too large for it (or NaN).
+// Returns their largest magnitude.
+__device__ __forceinline__ float store_split4(half_t* dst, size_t lo, float4 v, int* overflow) {
   if (!(fabsf(v.x) <= kSplitMax && fabsf(v.y) <= kSplitMax && fabsf(v.z) <= kSplitMax && fabsf(v.w) <= kSplitMax))
     *overflow = 1;
   half_t h[4], l[4];
@@ -23,16 +24,19 @@ __device__ __forceinline__ void store_split4(half_t* dst, size_t lo, float4 v, i
   split_f16(v.w, h[3], l[3]);
   *reinterpret_cast<half4*>(dst) = half4{h[0], h[1], h[2], h[3]};
   *reinterpret_cast<half4*>(dst + lo) = half4{l[0], l[1], l[2], l[3]};
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
 // cpu_layernorm (tokenizer_tests.cpp:2992-3010), one wave per row, the row in
 // registers: two passes over them, eps 1e-5.
 constexpr int kLnRows = 4;  // rows (waves) per block
 __global__ __launch_bounds__(kLnRows * 64) void ln_rows_kernel(const float* x, const float* g, const float* b, int M,
-                                                               half_t* y, size_t y_lo, int* overflow) {
+                                                               half_t* y, size_t y_lo, int* overflow,
+                                                               uint32_t* small, int sets, int stride) {
   constexpr int CH = kGptW / 256;  // float4 chunks per lane
   const int m = blockIdx.x * kLnRows + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (m >= M) return;
+  for (int i = lane; i < sets; i += 64) small[(size_t)i * stride + m] = 0u;
   float4 v[CH], gv[CH], bv[CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) v[c] = reinterpret_cast<const float4*>(x + (size_t)m * kGptW)[lane + 64 * c];
@@ -52,12 +56,14 @@ __global__ __launch_bounds__(kLnRows * 64) void ln_rows_kernel(const float* x, c
     q += (v[c].x * v[c].x + v[c].y * v[c].y) + (v[c].z * v[c].z + v[c].w * v[c].w);
   }
   const float inv = 1.0f / sqrtf(warp_sum(q) * (1.0f / kGptW) + 1e-5f);
+  float big = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c)
-    store_split4(y + (size_t)m * kGptW + 4 * (lane + 64 * c), y_lo,
-                 make_float4(v[c].x * inv * gv[c].x + bv[c].x, v[c].y * inv * gv[c].y + bv[c].y,
-                             v[c].z * inv * gv[c].z + bv[c].z, v[c].w * inv * gv[c].w + bv[c].w),
-                 overflow);
+    big = fmaxf(big, store_split4(y + (size_t)m * kGptW + 4 * (lane + 64 * c), y_lo,
+                                  make_float4(v[c].x * inv * gv[c].x + bv[c].x, v[c].y * inv * gv[c].y + bv[c].y,
+                                              v[c].z * inv * gv[c].z + bv[c].z, v[c].w * inv * gv[c].w + bv[c].w),
+                                  overflow));
+  if (__any(big > 0.f) && !__any(big >= kSplitFull)) *overflow = 1;
 }
 
 // Block (head, 16 queries); its four waves take alternate 16-key tiles with a
@@ -75,7 +81,7 @@ constexpr int kAttnWaves = 4;
 constexpr int kOStride = kHD + 4;  // LDS row of a query's output (floats)
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_rows_kernel(const float* q, const float* kc, const float* vc,
                                                                     int cap, int kv0, int M, half_t* y, size_t y_lo,
-                                                                    int* overflow) {
+                                                                    int* overflow, uint32_t* small) {
   __shared__ float sO[kAttnWaves][16][kOStride];
   __shared__ float sM[kAttnWaves][16], sL[kAttnWaves][16];
   const int h = blockIdx.x;
@@ -168,25 +174,29 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_rows_kernel(const float*
     L += f * sL[w][qi];
     O.x += f * ow.x; O.y += f * ow.y; O.z += f * ow.z; O.w += f * ow.w;
   }
-  store_split4(y + (size_t)(q0 + qi) * kGptW + h * kHD + d4, y_lo, make_float4(O.x / L, O.y / L, O.z / L, O.w / L),
-               overflow);
+  const float big = store_split4(y + (size_t)(q0 + qi) * kGptW + h * kHD + d4, y_lo,
+                                 make_float4(O.x / L, O.y / L, O.z / L, O.w / L), overflow);
+  // (16 lanes a query: one head's part of its row)
+  const uint32_t full = (uint32_t)(__ballot(big >= kSplitFull) >> (lane & 48)) & 0xffffu;
+  const uint32_t some = (uint32_t)(__ballot(big > 0.f) >> (lane & 48)) & 0xffffu;
+  if (!full && lr == 0) count_small(small + q0 + qi, kHeads, some != 0, overflow);
 }
 
 }  // namespace
 
 hipError_t launch_gpt_ln_rows(const float* x, const float* g, const float* b, int M, half_t* y, size_t y_lo,
-                              int* overflow, hipStream_t s) {
+                              int* overflow, hipStream_t s, uint32_t* small, int sets, int stride) {
   if (M <= 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(ln_rows_kernel, dim3((M + kLnRows - 1) / kLnRows), dim3(kLnRows * 64), 0, s, x, g, b, M, y, y_lo,
-                     overflow);
+                     overflow, small, sets, stride);
   return hipGetLastError();
 }
 
 hipError_t launch_gpt_attn_rows(const float* q, const float* kc, const float* vc, int cap, int kv0, int M,
-                                half_t* y, size_t y_lo, int* overflow, hipStream_t s) {
+                                half_t* y, size_t y_lo, int* overflow, uint32_t* small, hipStream_t s) {
   if (M <= 0 || kv0 < 0 || kv0 + M > cap) return hipErrorInvalidValue;
   hipLaunchKernelGGL(attn_rows_kernel, dim3(kHeads, (M + 15) / 16), dim3(kAttnWaves * 64), 0, s, q, kc, vc, cap, kv0,
-                     M, y, y_lo, overflow);
+                     M, y, y_lo, overflow, small);
   return hipGetLastError();
 }
 

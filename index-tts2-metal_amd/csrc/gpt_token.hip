@@ -84,6 +84,7 @@ struct Lds {  // (the small arrays first: LDS instructions hold 64 KB offsets)
   float o[4 * kAW][kHD];
   float ml[4 * kAW][2];
   float stat[2][kXW][2];  // (mean, sum of squared deviations) of equal parts of x
+  int holds[4][kPW];      // what each poll wave's part of a phase's input holds
   alignas(1024) float k[kLdsKeys * kHD];
   float v[kLdsKeys * kHD];
 };
@@ -223,10 +224,15 @@ __device__ __forceinline__ void all_stats(const Lds& s, int set, float& mean, fl
   const float var = (q + d * (float)kPoll) * (1.0f / kW);
   inv = 1.0f / sqrtf(var + 1e-5f);
 }
+// What a wave's part of a phase's input vector holds (big: a lane's largest
+// magnitude): 1 a nonzero value, 2 one of at least kSplitFull as well; uniform.
+__device__ __forceinline__ int holds(float big) {
+  return (__any(big > 0.f) ? 1 : 0) | (__any(big >= kSplitFull) ? 2 : 0);
+}
 // v[0], v[1], ... as split pairs at positions i, i + 1, i + step, i + step + 1, ...;
-// reports values that do not fit (or a NaN).
+// reports values that are too large (or a NaN).  Returns the largest magnitude.
 template <int N>
-__device__ __forceinline__ void put_split(half_t* hi, half_t* lo, int i, int step, const float (&v)[N], GptState* st) {
+__device__ __forceinline__ float put_split(half_t* hi, half_t* lo, int i, int step, const float (&v)[N], GptState* st) {
   float big = 0.f;
   bool nan = false;
 #pragma unroll
@@ -240,6 +246,7 @@ __device__ __forceinline__ void put_split(half_t* hi, half_t* lo, int i, int ste
     *reinterpret_cast<half2v*>(lo + i + (e / 2) * step) = half2v{l0, l1};
   }
   if (nan || big > kSplitMax) st->unfit = 1;
+  return big;
 }
 
 template <typename T>
@@ -617,19 +624,36 @@ __device__ __forceinline__ void poll_waves(const TokenArgs& a, Lds& s, int wg, i
       for (int i = 0; i < N; ++i) v[i] = (v[i] - mean) * inv * gv[i] + bv[i];
     }
   };
+  // The four phases' input vectors a layer, each in parts of a wave.  While the
+  // products run, between the phase's two barriers, every wave notes what its part
+  // holds, and after them wave 0 reports a vector that is all below kSplitFull
+  // (but not all 0).
+  float big = 0.f;
+  auto input_done = [&](int phase) {
+    lds_barrier();
+    const int h = holds(big);
+    if (lane == 0) s.holds[phase][pw] = h;
+    lds_barrier();
+    if (pw == 0) {
+      const int hp = lane < kPW ? s.holds[phase][lane] : 0;
+      if (__any(hp != 0) && !__any((hp & 2) != 0)) a.st->unfit = 1;
+    }
+  };
   auto put_x = [&]() {
+    big = 0.f;
     if (!xw) return;
-    bool fits = true;
+    bool nan = false;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       if (!ok(i)) continue;
-      fits = fits && fabsf(v[i]) <= kSplitMax;
+      nan = nan || !(v[i] == v[i]);
+      big = fmaxf(big, fabsf(v[i]));
       half_t h, l;
       split_f16(v[i], h, l);
       s.x[0][pos(i / 2) + (i & 1)] = h;
       s.x[1][pos(i / 2) + (i & 1)] = l;
     }
-    if (!fits) a.st->unfit = 1;
+    if (nan || big > kSplitMax) a.st->unfit = 1;
   };
   for (int i = lane + 64 * pw; i < 3 * kR3W - kW; i += 64 * kPW) s.x[0][kW + i] = s.x[1][kW + i] = (half_t)0.f;
   for (int i = lane + 64 * pw; i < 3 * kR3F - kMLP; i += 64 * kPW) s.xf[0][kMLP + i] = s.xf[1][kMLP + i] = (half_t)0.f;
@@ -647,8 +671,7 @@ __device__ __forceinline__ void poll_waves(const TokenArgs& a, Lds& s, int wg, i
       if (xw && slot[i / 2] == wg && ok(i)) s.xr[2 * third[i / 2] + (i & 1)] = v[i];
     norm(0);
     put_x();
-    lds_barrier();
-    lds_barrier();
+    input_done(0);
     // the head's query, and the new key and value: waves 0 (q, k) and 1 (v)
     if (wg < kAttnWG) {
       const int h = wg % kHeads, sp = wg / kHeads;
@@ -700,16 +723,14 @@ __device__ __forceinline__ void poll_waves(const TokenArgs& a, Lds& s, int wg, i
         t[2 * (i >> 2)] += c * o[2 * i];
         t[2 * (i >> 2) + 1] += c * o[2 * i + 1];
       }
-      put_split(s.x[0], s.x[1], (hb + hh) * kHD + d, kHD, t, a.st);
+      big = put_split(s.x[0], s.x[1], (hb + hh) * kHD + d, kHD, t, a.st);
     }
-    lds_barrier();
-    lds_barrier();
+    input_done(1);
     // c_fc's input
     if (xw) poll<NP, kSleepXb>(a.mail->xb, sizeof a.mail->xb, pairs, tag, v, dead, a);
     norm(1);
     put_x();
-    lds_barrier();
-    lds_barrier();
+    input_done(2);
     // the mlp projection's input
     {
       const int p0 = pw * 32 * NF + lane, f0 = 2 * p0;  // pairs p0 + 64 i, ten a slot
@@ -721,17 +742,15 @@ __device__ __forceinline__ void poll_waves(const TokenArgs& a, Lds& s, int wg, i
             return 8 * (kTokFSlot * sl + 2 * (p - sl * (kRF / 2)));
           },
           tag, f, dead, a);
-      put_split(s.xf[0], s.xf[1], f0, 128, f, a.st);
+      big = put_split(s.xf[0], s.xf[1], f0, 128, f, a.st);
     }
-    lds_barrier();
-    lds_barrier();
+    input_done(3);
   }
   if (xw) poll<NP, kSleepXa>(a.mail->xa, sizeof a.mail->xa, pairs, tag0 + a.L - 1, v, dead, a);
   norm(0);
   norm(1);
   put_x();
-  lds_barrier();
-  lds_barrier();
+  input_done(2);
 }
 
 // ----------------------------------------------------------------- key wave

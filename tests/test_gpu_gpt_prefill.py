@@ -4,8 +4,8 @@ LayerNorm and attention kernels.
 
 The reference is the same call with MIT2CFM_GPT_ROW_PREFILL=1: one row at a time
 through the decode step's fp32 kernels, which test_gpu_gpt.py holds to the
-oracle.  Both forms sum in fp32 (a split pair holds a value to 2^-22, and the
-weights are exact in f16), so they differ by the order of fp32 sums: logits of
+oracle.  Both forms sum in fp32 (a split pair holds a value to 2^-23, or 2^-36
+below 2^-13, and the weights are exact in f16), so they differ by the order of fp32 sums: logits of
 magnitude about 1 over sums of 1,280 and 5,120 terms, a few 1e-6 measured; the
 bar is test_gpu_gpt.py's 1e-5 for the same comparison.
 
@@ -162,5 +162,51 @@ def test_past_f16_the_prefix_goes_in_chunks(mit2, tensors, gpt2_t, monkeypatch, 
         ms = [min(r["prefill_ms"] for r in rs) for rs in (got, ref)]  # (the first with its attempt)
         print(f"P={P}: chunks {ms[0]:.2f} ms, rows {ms[1]:.2f} ms", flush=True)
         assert P < 100 or ms[0] < 0.55 * ms[1]
+    finally:
+        c.close()
+
+
+def small_values(gpt2_t, where, spare=False):
+    """Weights whose layer-1 inputs of one product are all about 2^-16 (fp32 biases
+    and LayerNorm weights; that product's weights are raised, so they matter), or
+    all but one of them (`spare`)."""
+    t = dict(gpt2_t)
+
+    def arr(name, shape):
+        t["gpt.gpt.h.1." + name] = a = np.array(t["gpt.gpt.h.1." + name], np.float32).reshape(shape)
+        return a
+
+    noise = (np.random.default_rng(6).uniform(0.5, 1.0, 5120) * 2.0**-16).astype(np.float32)
+    if where == "layernorm":
+        arr("ln_2.weight", -1)[:] = 0
+        v, w = arr("ln_2.bias", -1), arr("mlp.c_fc.weight", (W, 5120))
+    elif where == "value":
+        arr("attn.c_attn.weight", (W, 3 * W))[:, 2 * W :] = 0
+        v, w = arr("attn.c_attn.bias", -1)[2 * W :], arr("attn.c_proj.weight", (W, W))
+    else:
+        arr("mlp.c_fc.weight", (W, 5120))[:] = 0
+        v, w = arr("mlp.c_fc.bias", -1), arr("mlp.c_proj.weight", (5120, W))
+    v[:] = noise[: v.size]
+    if spare:
+        v[3] = 0.5
+    w *= 2.0**12
+    return t
+
+
+@pytest.mark.parametrize("where", ["layernorm", "value", "gelu"])
+@pytest.mark.parametrize("spare", [False, True])
+def test_rows_below_a_pairs_full_precision(mit2, tensors, gpt2_t, monkeypatch, where, spare):
+    """A pair holds values below 2^-13 to 2^-36 only.  A product whose input row
+    is all that small runs plain (the same bits as asking for it); one with a
+    single larger value keeps its row products, which then hold the row to 2^-23
+    of that value."""
+    c = mit2.Context({**tensors, **small_values(gpt2_t, where, spare)}, device=0)
+    try:
+        for M in (2, 70, 300):
+            print(f"small {where} spare={spare} M={M}", flush=True)
+            got, ref = _both(c, _rows(M, 9), monkeypatch, fits=spare)
+            for a, b in zip(got[:3], ref[:3]):
+                assert np.isfinite(a).all()
+                assert np.abs(a - b).max() <= 1e-5 if spare else np.array_equal(a, b)
     finally:
         c.close()

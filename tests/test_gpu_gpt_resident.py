@@ -3,7 +3,7 @@
 The reference is the same call on a context created with MIT2CFM_GPT_RESIDENT=0,
 whose steps are separate fp32 launches that test_gpu_gpt.py holds to the oracle.
 The resident kernel's products are split f16 pairs on the matrix cores (a pair
-holds a value to 2^-22, the weights are exact in f16) with fp32 sums, so the two
+holds a value to 2^-23, or 2^-36 below 2^-13, the weights are exact in f16) with fp32 sums, so the two
 differ by the order of fp32 sums of up to 5,120 terms: logits of magnitude about
 1 agree to a few 1e-6, and the bar is test_gpu_gpt.py's 1e-5 for such pairs.
 
@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 
 from conftest import gpt_paths
+from test_gpu_gpt_prefill import small_values
 
 pytestmark = pytest.mark.gpu
 
@@ -185,6 +186,21 @@ def test_decode_values_past_f16(mit2, tensors, monkeypatch, where):
             assert ra["predicted"].tolist() == rb["predicted"].tolist()
             assert np.isfinite(ra["last_logits"]).all()
             assert np.array_equal(ra["last_logits"], rb["last_logits"])
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("where", ["layernorm", "value", "gelu"])
+@pytest.mark.parametrize("spare", [False, True])
+def test_steps_below_a_pairs_full_precision(mit2, tensors, monkeypatch, where, spare):
+    """As test_rows_below_a_pairs_full_precision, for the token steps."""
+    t = small_values(_tensors(mit2, tensors, 2), where, spare)
+    a, b = mit2.Context(t, device=0), _plain(mit2, t, monkeypatch)
+    try:
+        ra, how = gpt_paths(a, lambda: a.gpt_kv_greedy(_rows(0, 0), 6))
+        assert how == ({"resident_steps": 6} if spare else {"range_reruns": 1, "plain_steps": 6})
+        _same(ra, b.gpt_kv_greedy(_rows(0, 0), 6))
     finally:
         a.close()
         b.close()
