@@ -1096,7 +1096,9 @@ void launch_gemv(const GemvArgs& a, hipStream_t s) {
 template <int LPR, int WAVES, int UR>
 constexpr int rows_of() { return WAVES * (64 / LPR) * UR; }
 constexpr int head_blocks() { return (kVocab + rows_of<GPT_HEAD_SHAPE>() - 1) / rows_of<GPT_HEAD_SHAPE>(); }
-static_assert(head_blocks() <= 4096, "argmax_kernel reduces at most 4096 block maxima");
+// Block maxima of either head: the plain one's blocks, the resident kernel's workgroups.
+constexpr int kHeadMaxima = std::max(head_blocks(), kTokWG);
+static_assert(kHeadMaxima <= 4096, "argmax_kernel reduces at most 4096 block maxima");
 
 void launch_qkv(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_QKV_SHAPE, PRO_LN, EPI_QKV>(a, s); }
 void launch_attn_proj(const GemvArgs& a, hipStream_t s) { launch_gemv<kW, GPT_PROJ_SHAPE, PRO_PLAIN, EPI_RES>(a, s); }
@@ -1320,8 +1322,8 @@ struct GptDecoder::Impl {
     const size_t f = sizeof(float);
     size_t bytes = align256(sizeof(GptState)) + align256((size_t)pred_cap * 4) +
                    align256(((size_t)pred_cap + 1) * 4) + 3 * align256(kW * f) + align256(kMLP * f) +
-                   align256(kVocab * f) + 2 * align256(kW * f) + align256((size_t)head_blocks() * f) +
-                   align256((size_t)head_blocks() * 4) +
+                   align256(kVocab * f) + 2 * align256(kW * f) + align256((size_t)kHeadMaxima * f) +
+                   align256((size_t)kHeadMaxima * 4) +
                    3 * align256((size_t)chunk_cap * kW * f) + align256((size_t)chunk_cap * kMLP * f) +
                    align256((size_t)kPlainRows * kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
@@ -1338,8 +1340,8 @@ struct GptDecoder::Impl {
     logits = static_cast<float*>(ws.take(kVocab * f));
     lnf = static_cast<float*>(ws.take(kW * f));
     fn = static_cast<float*>(ws.take(kW * f));
-    blk_val = static_cast<float*>(ws.take((size_t)head_blocks() * f));
-    blk_idx = static_cast<int*>(ws.take((size_t)head_blocks() * 4));
+    blk_val = static_cast<float*>(ws.take((size_t)kHeadMaxima * f));
+    blk_idx = static_cast<int*>(ws.take((size_t)kHeadMaxima * 4));
     xr = static_cast<float*>(ws.take((size_t)chunk_cap * kW * f));
     qr = static_cast<float*>(ws.take((size_t)chunk_cap * kW * f));
     a16 = static_cast<half_t*>(ws.take((size_t)chunk_cap * kW * 2 * sizeof(half_t)));
@@ -1410,6 +1412,7 @@ struct GptDecoder::Impl {
 
   // The next token from the logits (nb: workgroups that left a maximum).
   void enqueue_pick(bool sample, int nb) {
+    if (nb > kHeadMaxima) GPT_OK(hipErrorInvalidValue);
     if (sample)
       hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
                          hist);
