@@ -35,11 +35,13 @@
 //   waves 0-9    products.  Wave w takes the K slice [K w / 10, K (w + 1) / 10)
 //                of all the workgroup's rows; the partial sums meet in LDS and
 //                wave 0 finishes them
-//   waves 10-13  poll the phase's input vector into LDS (with the LayerNorm
-//                statistics of each wave's 320 values); the attention's
-//                arithmetic (80 workgroups: 20 heads in 4 parts)
-//   waves 14-15  bring the LayerNorm weights and biases, and the keys and values
-//                of the workgroup's part of a head, into LDS a layer ahead
+//   waves 10-14  poll the phase's input vector into LDS (the residual stream four
+//                of them, with the LayerNorm statistics of each wave's 320
+//                values); four do the attention's arithmetic (80 workgroups: 20
+//                heads in 4 parts)
+//   wave 15      brings the LayerNorm weights and biases, the products' biases and
+//                the keys and values of the workgroup's part of a head into LDS a
+//                layer ahead
 #include "gpt_token.h"
 
 #include <type_traits>
@@ -88,6 +90,8 @@ struct Lds {  // (the small arrays first: LDS instructions hold 64 KB offsets)
   alignas(1024) float k[kLdsKeys * kHD];
   float v[kLdsKeys * kHD];
 };
+// (a larger one would not launch, and every step would silently be plain)
+static_assert(sizeof(Lds) <= 160 * 1024, "the LDS of a CU");
 
 // LDS barrier: orders this wave's LDS accesses only (a full fence would also
 // wait for the weights in flight).
