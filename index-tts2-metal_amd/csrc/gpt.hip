@@ -404,6 +404,65 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
   }
 }
 
+// Room for other work beside the resident step kernel, which holds every CU: left
+// alone it runs step after step, and another stream's kernels get only the gaps
+// between two of them (a mel decode of 128 frames took 158 ms beside a greedy
+// call instead of 6).  The kernel's workgroups start within 0.85 us of each other
+// on a free GPU (15,000 steps) and some microseconds apart where another kernel
+// holds CUs (more than 1.5 us in 85 to 95 of 100 steps; two steps after such a
+// one count too), and that tells.  While it does, each step owes the others
+// twice its time, and once 2.3 ms are owed the pick behind a step waits them off:
+// its one CU apart the GPU is free.  Beside it (256 codes after 150 rows, alone
+// 104 ms; plain launches, which share the GPU by themselves, in brackets):
+//   mel decode, 860 frames   greedy 307 ms [317]  a decode 35.5 ms [31.7], alone 21.6
+//   mel decode, 128 frames          304 [265]              9.9 [9.6], 6.0
+//   vocoder, 861 frames             348 [437]              9.0 [7.7], 6.2
+//   condition, 553 codes            303 [255]              0.15 [0.13], 0.10
+// (2.5 times: 358 and 33.6 in the first row; waits after every step: 311 and 38.8,
+// as the others then refill the caches each time).
+constexpr int kYieldSpread = 150, kYieldSteps = 3;  // ticks of 10 ns; steps a sign counts for
+constexpr uint32_t kYieldShare = 2, kYieldLeast = 230000, kYieldMost = 800000;
+constexpr int kYieldLooks = 20000;  // bound of the wait, about 1 us each
+constexpr int kYieldWave = 15;      // of the pick kernels' 16
+// The yield wave's share of the workgroups' start times, read ahead.
+struct StartTicks {
+  uint32_t t[kTokWG / 64];
+};
+__device__ __forceinline__ StartTicks start_ticks(const uint32_t* start) {
+  StartTicks s = {};
+  if (start && (int)(threadIdx.x >> 6) == kYieldWave)
+#pragma unroll
+    for (int i = 0; i < kTokWG / 64; ++i) s.t[i] = start[(threadIdx.x & 63) + 64 * i];
+  return s;
+}
+// `start` is NULL behind the plain launches.
+__device__ __forceinline__ void yield_gpu(GptState* st, const uint32_t* start, const StartTicks& s) {
+  if (!start || (int)(threadIdx.x >> 6) != kYieldWave) return;
+  const uint32_t t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s.t[0]);
+  int first = 0, last = 0;  // (against workgroup 0's: the clock may wrap)
+#pragma unroll
+  for (int i = 0; i < kTokWG / 64; ++i) {
+    first = min(first, (int)(s.t[i] - t0));
+    last = max(last, (int)(s.t[i] - t0));
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    first = min(first, __shfl_xor(first, off, kWave));
+    last = max(last, __shfl_xor(last, off, kWave));
+  }
+  const uint32_t now = device_ticks(), took = now - t0 - (uint32_t)first;
+  int left = st->yield_left;
+  if (last - first > kYieldSpread) left = kYieldSteps;
+  uint32_t owed = left > 0 ? min(st->owed + took * kYieldShare, kYieldMost) : 0u;
+  const bool now_due = owed >= kYieldLeast;
+  if ((threadIdx.x & 63) == 0) {
+    st->yield_left = max(left - 1, 0);
+    st->owed = now_due ? 0u : owed;
+  }
+  if (now_due)
+    for (int i = 0; i < kYieldLooks && device_ticks() - now < owed; ++i) __builtin_amdgcn_s_sleep(32);
+}
+
 // The do_sample path of the decode loop (run_gpt_kv_greedy_metal with
 // sampling, gpt.cpp:2221-2240): apply_gpt_sampling_processors (:1618-1718) to
 // the step's logits over the history (the caller's repetition_history_prefix,
@@ -437,8 +496,10 @@ __device__ __forceinline__ double sm64_unit(uint64_t& s) {
 
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* logits, GptState* st,
                                                                 uint32_t* predicted, uint32_t* inputs,
-                                                                float* proc, const uint32_t* hist_prefix) {
+                                                                float* proc, const uint32_t* hist_prefix,
+                                                                const uint32_t* start) {
   if (st->stopped) return;
+  const StartTicks ticks = start_ticks(start);
   if (st->failed()) {  // the host takes the step again
     if (threadIdx.x == 0) st->stopped = 1;
     return;
@@ -731,6 +792,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
     // back from memory, took 12 us more of a code's 430.)
     for (int i = tid; i < (N + 31) / 32; i += kSampleThreads) seen[i] = 0u;  // now: removed by top-p
     __syncthreads();
+    yield_gpu(st, start, ticks);
     if (tid >= 64) return;
     const uint32_t idx = tid < m ? lidx[tid] : 0u;
     const bool finite = tid < m && proc[idx] != -INFINITY;  // (ahead of top-p's stores)
@@ -774,6 +836,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* log
     return;
   }
   __syncthreads();
+  yield_gpu(st, start, ticks);
   if (tid != 0) return;
   // survivors in index order: (index, its exp) -- removed ones are skipped
   auto index_walk = [&](auto&& f) {
@@ -833,8 +896,9 @@ __global__ void advance_rows_kernel(GptState* st) {
 // stop at the stop token, else append it to the inputs.
 __global__ __launch_bounds__(1024) void argmax_kernel(const float* blk_val, const int* blk_idx, int nb,
                                                       GptState* st, uint32_t* predicted, uint32_t* inputs,
-                                                      int check_stop) {
+                                                      int check_stop, const uint32_t* start) {
   if (check_stop && st->stopped) return;
+  const StartTicks ticks = start_ticks(start);
   if (check_stop && st->failed()) {  // the host takes the step again
     if (threadIdx.x == 0) st->stopped = 1;
     return;
@@ -864,6 +928,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* blk_val, cons
   }
   if (lane == 0) { wv[wave] = bv; wi[wave] = bi; }
   __syncthreads();
+  yield_gpu(st, start, ticks);
   if (tid != 0) return;
   for (int w2 = 1; w2 < 16; ++w2)
     if (wv[w2] > bv || (wv[w2] == bv && wi[w2] < bi)) { bv = wv[w2]; bi = wi[w2]; }
@@ -1180,6 +1245,7 @@ struct GptDecoder::Impl {
   float* proc = nullptr;        // the sampler's processed logits [8194]
   uint32_t* hist = nullptr;     // the repetition-history prefix [kMaxHistory]
   TokenMail* mail = nullptr;    // the resident step kernel's words
+  uint32_t* start = nullptr;    //   and its workgroups' start times
   uint32_t epoch = 1;           // first tag epoch no launch has used
   float* part = nullptr;        // attention splits: [8 query rows][20 heads][nsplit_max][66]
   int nsplit_max = 0;
@@ -1328,6 +1394,7 @@ struct GptDecoder::Impl {
                    align256((size_t)kPlainRows * kHeads * (cap / kChunk) * kPartF * f) + align256(kVocab * f) +
                    2 * align256((size_t)L * cap * kW * f) + align256((size_t)rows_cap * kW * f) +
                    align256((size_t)GptDecoder::kMaxHistory * 4) + align256(sizeof(TokenMail)) +
+                   align256(kTokWG * 4) +
                    align256((size_t)2 * L * chunk_cap * 4);
     ws.reserve(bytes);
     st = static_cast<GptState*>(ws.take(sizeof(GptState)));
@@ -1351,6 +1418,7 @@ struct GptDecoder::Impl {
     nsplit_max = cap / kChunk;
     mail = static_cast<TokenMail*>(ws.take(sizeof(TokenMail)));
     GPT_OK(hipMemsetAsync(mail, 0, sizeof(TokenMail), s));  // no word carries a tag yet
+    start = static_cast<uint32_t*>(ws.take(kTokWG * 4));
     row_small = static_cast<uint32_t*>(ws.take((size_t)2 * L * chunk_cap * 4));
     epoch = 1;
     part = static_cast<float*>(ws.take((size_t)kPlainRows * kHeads * nsplit_max * kPartF * f));
@@ -1405,19 +1473,21 @@ struct GptDecoder::Impl {
     a.lnf_w = lnf_w; a.lnf_b = lnf_b; a.fn_w = fn_w; a.fn_b = fn_b; a.head_b = head_b; a.head_w = head_w;
     a.mel_emb = mel_emb; a.pos_emb = pos_emb;
     a.st = st; a.kc = kc; a.vc = vc; a.cap = cap; a.mail = mail;
-    a.logits = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.spin_limit = spin_limit;
+    a.logits = logits; a.blk_val = blk_val; a.blk_idx = blk_idx; a.start = start; a.spin_limit = spin_limit;
     GPT_OK(launch_gpt_token(a, s));
-    enqueue_pick(sample, kTokWG);
+    enqueue_pick(sample, kTokWG, start);
   }
 
-  // The next token from the logits (nb: workgroups that left a maximum).
-  void enqueue_pick(bool sample, int nb) {
+  // The next token from the logits (nb: workgroups that left a maximum; begun:
+  // when the resident kernel's started).
+  void enqueue_pick(bool sample, int nb, const uint32_t* begun = nullptr) {
     if (nb > kHeadMaxima) GPT_OK(hipErrorInvalidValue);
     if (sample)
       hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, logits, st, predicted, inputs, proc,
-                         hist);
+                         hist, begun);
     else
-      hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, nb, st, predicted, inputs, 1);
+      hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, blk_val, blk_idx, nb, st, predicted, inputs, 1,
+                         begun);
     GPT_OK(hipGetLastError());
   }
 
@@ -1947,7 +2017,7 @@ const char* GptDecoder::profile_launch(int kernel, int launches, double* bytes) 
         a.check_stop = 0;
         launch_head(a, d.s);
         hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, d.s, d.blk_val, d.blk_idx, head_blocks(), d.st,
-                           d.predicted, d.inputs, 0);
+                           d.predicted, d.inputs, 0, static_cast<const uint32_t*>(nullptr));
         break;
       default:
         d.launch_attention(d.q, d.kc + (size_t)(i % d.L) * d.cap * kW, d.vc + (size_t)(i % d.L) * d.cap * kW,

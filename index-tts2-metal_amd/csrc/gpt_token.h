@@ -39,8 +39,18 @@ struct TokenArgs {
   float* logits;
   float* blk_val;  // [kTokWG] first maximum of each workgroup's logits and its row
   int* blk_idx;
+  uint32_t* start;  // [kTokWG] when each workgroup started (device_ticks)
   uint32_t spin_limit;  // polls a wait may take (a million: about a second)
 };
+
+// The device's constant clock: ticks of 10 ns.
+__device__ __forceinline__ uint32_t device_ticks() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__builtin_amdgcn_s_memrealtime();
+#else
+  return 0;
+#endif
+}
 
 // Whether every workgroup of the kernel fits the device at once.
 bool gpt_token_fits(int device);

@@ -844,6 +844,7 @@ __global__ __launch_bounds__(kThreads) void token_kernel(TokenArgs a) {
   if (a.st->stopped) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wg = blockIdx.x;
+  if (threadIdx.x == kThreads - 1) a.start[wg] = device_ticks();
   const int kv = __builtin_amdgcn_readfirstlane(a.st->kv);
   const uint32_t tag0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)((a.st->epoch + (uint32_t)a.st->step) << 6));
   if (wave < kCW)

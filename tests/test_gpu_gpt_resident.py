@@ -14,6 +14,7 @@ lengths run over every remainder of 4, from empty, and across 832.
 from __future__ import annotations
 
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -139,6 +140,53 @@ def test_contexts_on_threads_take_turns(mit2, tensors):
     finally:
         for c in ctx:
             c.close()
+
+
+def test_other_work_beside_a_decode(mit2, tensors):
+    """Mel decodes on a second context while the resident kernel, which holds the
+    whole GPU, makes codes on the first: both give what they give alone, no step
+    is taken plain, and the mel decodes get their part of the GPU (measured 1.6 of
+    their time alone; 26 when the steps followed each other without a pause)."""
+    t = _tensors(mit2, tensors, 24)
+    a, b = mit2.Context(t, device=0), mit2.Context(tensors, device=0)
+    try:
+        rng = np.random.default_rng(8)
+        args = [rng.standard_normal(s).astype(np.float32) for s in ((128, 80), (38, 80), (128, 512), (192,))]
+        x = _rows(150, 9)
+        mel = lambda: b.decode(*args, 12, 0.7)
+
+        def seconds(n=10):
+            t0 = time.perf_counter()
+            for _ in range(n):
+                assert np.array_equal(mel(), mel0)
+            return (time.perf_counter() - t0) / n
+
+        mel0, codes0 = mel(), a.gpt_kv_greedy(x, 400)
+        alone = seconds()
+        before, stop, got = a.gpt_counts(), threading.Event(), []
+
+        def work():
+            while not stop.is_set():
+                got.append(a.gpt_kv_greedy(x, 400))
+
+        th = threading.Thread(target=work)
+        th.start()
+        try:
+            beside = seconds(30)
+        finally:
+            stop.set()
+            th.join()
+        print(f"mel decode alone {1e3 * alone:.2f} ms, beside codes {1e3 * beside:.2f} ms", flush=True)
+        for g in got:
+            assert g["predicted"].tolist() == codes0["predicted"].tolist()
+            assert np.array_equal(g["last_logits"], codes0["last_logits"])
+        n = a.gpt_counts()
+        assert n["resident_steps"] - before["resident_steps"] == 400 * len(got)
+        assert n["plain_steps"] == n["wait_reruns"] == n["range_reruns"] == 0
+        assert beside <= 4 * alone
+    finally:
+        a.close()
+        b.close()
 
 
 def test_a_wait_that_runs_out_falls_back(mit2, tensors, monkeypatch):
