@@ -84,7 +84,6 @@ struct GemmArgs {
   int n_store = 0;  // if nonzero: only columns < n_store are stored (weights zero-padded to N)
   const half_t* A_zero = nullptr;  // A_CONVP: >= conv_c zero halves, read by the padding taps
   int conv_window = 1;             // A_CONVP with M = T: 0 streams every tap's rows (no A_CONVW)
-  int peers = 1;                   // A_CONVP: products in this one's launch (launch_gemm_group sets it)
   uint32_t conv_magic = 0;         // A_CONVW, set by launch_gemm: ceil(2^32 / conv_c), so that
                                    // k / conv_c = umulhi(k, conv_magic) for k conv_c < 2^32
   // weights

@@ -2046,10 +2046,8 @@ hipError_t launch_gemm_group(const GemmArgs* a, int n, AMode amode, EpiMode epi,
   HeldLaunch h[kMaxGroup];
   bool same = n == kMaxGroup;
   for (int i = 0; i < n; ++i) {
-    GemmArgs g = a[i];
-    g.peers = n;
     t_hold = &h[i];
-    const hipError_t e = launch_gemm(g, amode, epi, stream);
+    const hipError_t e = launch_gemm(a[i], amode, epi, stream);
     t_hold = nullptr;
     if (e != hipSuccess) return e;
     same = same && h[i].group && h[i].group == h[0].group && a[i].M == a[0].M && a[i].N == a[0].N;
