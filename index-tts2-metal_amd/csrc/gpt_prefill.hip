@@ -36,7 +36,6 @@ __global__ __launch_bounds__(kLnRows * 64) void ln_rows_kernel(const float* x, c
   constexpr int CH = kGptW / 256;  // float4 chunks per lane
   const int m = blockIdx.x * kLnRows + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (m >= M) return;
-  for (int i = lane; i < sets; i += 64) small[(size_t)i * stride + m] = 0u;
   float4 v[CH], gv[CH], bv[CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) v[c] = reinterpret_cast<const float4*>(x + (size_t)m * kGptW)[lane + 64 * c];
@@ -63,7 +62,8 @@ __global__ __launch_bounds__(kLnRows * 64) void ln_rows_kernel(const float* x, c
                                   make_float4(v[c].x * inv * gv[c].x + bv[c].x, v[c].y * inv * gv[c].y + bv[c].y,
                                               v[c].z * inv * gv[c].z + bv[c].z, v[c].w * inv * gv[c].w + bv[c].w),
                                   overflow));
-  if (__any(big > 0.f) && !__any(big >= kSplitFull)) *overflow = 1;
+  if (!__any(big >= kSplitFull) && __any(big > 0.f)) *overflow = 1;
+  for (int i = lane; i < sets; i += 64) small[(size_t)i * stride + m] = 0u;  // (last: nothing waits for it)
 }
 
 // Block (head, 16 queries); its four waves take alternate 16-key tiles with a
@@ -177,9 +177,11 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_rows_kernel(const float*
   const float big = store_split4(y + (size_t)(q0 + qi) * kGptW + h * kHD + d4, y_lo,
                                  make_float4(O.x / L, O.y / L, O.z / L, O.w / L), overflow);
   // (16 lanes a query: one head's part of its row)
-  const uint32_t full = (uint32_t)(__ballot(big >= kSplitFull) >> (lane & 48)) & 0xffffu;
-  const uint32_t some = (uint32_t)(__ballot(big > 0.f) >> (lane & 48)) & 0xffffu;
-  if (!full && lr == 0) count_small(small + q0 + qi, kHeads, some != 0, overflow);
+  const uint64_t full = __ballot(big >= kSplitFull) >> (lane & 48);
+  if ((full & 0xffffu) == 0) {
+    const uint64_t some = __ballot(big > 0.f) >> (lane & 48);
+    if (lr == 0) count_small(small + q0 + qi, kHeads, (some & 0xffffu) != 0, overflow);
+  }
 }
 
 }  // namespace
