@@ -409,18 +409,21 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
 // between two of them (a mel decode of 128 frames took 158 ms beside a greedy
 // call instead of 6).  The kernel's workgroups start within 0.85 us of each other
 // on a free GPU (15,000 steps) and some microseconds apart where another kernel
-// holds CUs (more than 1.5 us in 85 to 95 of 100 steps; two steps after such a
-// one count too), and that tells.  While it does, each step owes the others
-// twice its time, and once 2.3 ms are owed the pick behind a step waits them off:
-// its one CU apart the GPU is free.  Beside it (256 codes after 150 rows, alone
-// 104 ms; plain launches, which share the GPU by themselves, in brackets):
+// holds CUs (more than 1.5 us in 85 to 95 of 100 steps), and that tells: two such
+// steps close together, as a single one comes up by itself now and then (one in
+// 1,000 under a profiler).  From then on, and for two steps after the last sign,
+// each step owes the others twice its time, and once 2.3 ms are owed the pick
+// behind a step waits them off: its one CU apart the GPU is free.  Beside it
+// (256 codes after 150 rows, alone 104 ms; plain launches, which share the GPU by
+// themselves, in brackets):
 //   mel decode, 860 frames   greedy 307 ms [317]  a decode 35.5 ms [31.7], alone 21.6
 //   mel decode, 128 frames          304 [265]              9.9 [9.6], 6.0
 //   vocoder, 861 frames             348 [437]              9.0 [7.7], 6.2
 //   condition, 553 codes            303 [255]              0.15 [0.13], 0.10
 // (2.5 times: 358 and 33.6 in the first row; waits after every step: 311 and 38.8,
 // as the others then refill the caches each time).
-constexpr int kYieldSpread = 150, kYieldSteps = 3;  // ticks of 10 ns; steps a sign counts for
+constexpr int kYieldSpread = 150;                 // ticks of 10 ns
+constexpr int kYieldSign = 3, kYieldFull = 6;     // a sign's weight, which a step without one lowers by 1
 constexpr uint32_t kYieldShare = 2, kYieldLeast = 230000, kYieldMost = 800000;
 constexpr int kYieldLooks = 20000;  // bound of the wait, about 1 us each
 constexpr int kYieldWave = 15;      // of the pick kernels' 16
@@ -451,12 +454,12 @@ __device__ __forceinline__ void yield_gpu(GptState* st, const uint32_t* start, c
     last = max(last, __shfl_xor(last, off, kWave));
   }
   const uint32_t now = device_ticks(), took = now - t0 - (uint32_t)first;
-  int left = st->yield_left;
-  if (last - first > kYieldSpread) left = kYieldSteps;
-  uint32_t owed = left > 0 ? min(st->owed + took * kYieldShare, kYieldMost) : 0u;
+  int signs = st->yield_signs;
+  signs = last - first > kYieldSpread ? min(signs + kYieldSign, kYieldFull) : max(signs - 1, 0);
+  uint32_t owed = signs > kYieldSign ? min(st->owed + took * kYieldShare, kYieldMost) : 0u;
   const bool now_due = owed >= kYieldLeast;
   if ((threadIdx.x & 63) == 0) {
-    st->yield_left = max(left - 1, 0);
+    st->yield_signs = signs;
     st->owed = now_due ? 0u : owed;
   }
   if (now_due)

@@ -40,8 +40,8 @@ struct GptState {
   int32_t unfit;      // 1: a value of the resident step kernel did not fit one
   int32_t aborted;    // 1: a wait of the resident step kernel ran out
   int32_t pend;       // prefix rows the plain prefill's chunks cover (rows 0..pend-1)
-  int32_t yield_left; // steps that still leave the GPU to others for a while (gpt.hip, yield_gpu)
-  uint32_t owed;      // and the ticks owed to them
+  int32_t yield_signs;  // of other work on the GPU lately (gpt.hip, yield_gpu)
+  uint32_t owed;        // and the ticks owed to it
   int32_t pad[5];
 
   // The logits are worthless: no token is picked from them.
