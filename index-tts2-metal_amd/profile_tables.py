@@ -24,10 +24,10 @@ It reads whichever of these inputs exist and writes the summary each one feeds:
       rocprofv3 --pmc FETCH_SIZE (then WRITE_SIZE) -T --output-format csv -d RAW/pmc_bfetch -o fetch --
           python3 -u bench.py <short run, see BENCH_PMC>
     -> traffic_gemm_wavenet_conv_gate_T860.json
-  gpttrace/bench_kernel_trace.csv, gpttrace/bench_kernel_stats.csv, gpt_trace.log,
-  gptpmc_fetch/fetch_counter_collection.csv, gptpmc_write/write_counter_collection.csv
+  gpttrace/bench_kernel_trace.csv, gpttrace/bench_kernel_stats.csv,
+  gpt_trace.log, gptpmc_{fetch,write,sq}/{fetch,write,sq}_counter_collection.csv
       the same with MIT2CFM_GRAPH=0 and the GPT section of bench.py (see GPT_CMDS)
-    -> gpt_decode_P150_553codes_kernel_trace.md, traffic_gemv_gpt_c_fc.json
+    -> gpt_decode_P150_553codes_kernel_trace.md, traffic_gpt_token_kernel.json
 
 Any of these CSVs may come gzip-compressed (NAME.csv.gz); it is unpacked first.
 
@@ -43,6 +43,7 @@ import collections
 import csv
 import gzip
 import json
+import re
 import shutil
 from pathlib import Path
 
@@ -63,12 +64,14 @@ PMC_PASSES = {
 PMC_PROG = "python3 -u index-tts2-metal_amd/profile_kernels.py --launches 20"
 BENCH_PMC = ("python3 -u bench.py --steps 1 --warmup 1 --no-cpu-baseline --no-cpu-1thread --no-configs "
              "--kernel-launches 5 --voc-calls 0 --acoustic-calls 0 --cond-calls 1 --gpt-codes 0")
+GPT_SQ = "SQ_INSTS_MFMA SQ_INSTS_VALU SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_BUSY_CU_CYCLES"
 GPT_BENCH = ("python3 -u bench.py --steps 1 --warmup 1 --no-cpu-baseline --no-configs --kernel-launches 5 "
              "--voc-calls 0 --acoustic-calls 0 --cond-calls 1")
 GPT_CMDS = [
-    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --kernel-trace --stats -T --output-format csv -d $RAW/gpttrace -o bench -- {GPT_BENCH}",
-    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --pmc FETCH_SIZE -T --output-format csv -d $RAW/gptpmc_fetch -o fetch -- {GPT_BENCH}",
-    f"MIT2CFM_GRAPH=0 MIT2CFM_GPT_RESIDENT=0 rocprofv3 --pmc WRITE_SIZE -T --output-format csv -d $RAW/gptpmc_write -o write -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 rocprofv3 --kernel-trace --stats --output-format csv -d $RAW/gpttrace -o bench -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 rocprofv3 --pmc FETCH_SIZE --output-format csv -d $RAW/gptpmc_fetch -o fetch -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 rocprofv3 --pmc WRITE_SIZE --output-format csv -d $RAW/gptpmc_write -o write -- {GPT_BENCH}",
+    f"MIT2CFM_GRAPH=0 rocprofv3 --pmc {GPT_SQ} --output-format csv -d $RAW/gptpmc_sq -o sq -- {GPT_BENCH}",
 ]
 
 
@@ -583,9 +586,6 @@ Raw counters (per dispatch):
                 print("wrote traffic_gemm_wavenet_conv_gate_T860.json")
 
 
-GPT_WHAT = {"c_attn": "c_attn GEMV 3840x1280 + LN, K/V to cache", "attn_proj": "attn c_proj GEMV 1280x1280 + residual",
-            "c_fc": "c_fc GEMV 5120x1280 + LN + gelu_new", "mlp_proj": "mlp c_proj GEMV 1280x5120 + residual",
-            "mel_head": "mel_head GEMV 8194x1280 + ln_f + final_norm"}
 def gemv_roles(rows: list[dict], grid_key: str, wg_key: str) -> dict:
     """Kernel id -> product for the decode-step GEMVs, from their launch order
     within a layer (c_attn, the attention, attn c_proj, c_fc, mlp c_proj):
@@ -612,17 +612,23 @@ def gemv_roles(rows: list[dict], grid_key: str, wg_key: str) -> dict:
     return roles
 
 
-def gpt_kernel_key(r: dict, roles: dict) -> str:
+# The prefill's products by their epilogue (EpiMode in gemm.h).
+GPT_PREFILL_GEMM = {9: "c_fc + gelu_new", 10: "c_attn, K/V to cache", 11: "c_proj + residual"}
+
+
+def gpt_kernel_key(r: dict, roles: dict) -> str | None:
+    """The kernel's row in the GPT table; None for other stages' kernels."""
     n = r["Kernel_Name"]
-    for k in ("gemv_kernel", "attn_split_kernel", "attn_combine_kernel", "sample_kernel",
-              "embed_rows_kernel", "embed_kernel", "argmax_kernel", "advance_rows_kernel"):
+    for k in ("token_kernel", "gemv_rows_kernel", "gemv_kernel", "attn_split_kernel", "attn_combine_kernel",
+              "attn_rows_kernel", "ln_rows_kernel", "sample_kernel", "embed_rows_kernel", "embed_kernel",
+              "argmax_kernel", "advance_rows_kernel"):
         if k in n:
-            if k.startswith("gemv"):
+            if k == "gemv_kernel":
                 blocks = int(r["Grid_Size_X"]) // int(r["Workgroup_Size_X"])
-                role = roles.get(r["Kernel_Id"])
-                return f"{k} {role or '?'} (grid {blocks}x{r['Workgroup_Size_X']})"
+                return f"{k} {roles.get(r['Kernel_Id'], 'of the plain launches')} (grid {blocks}x{r['Workgroup_Size_X']})"
             return k
-    return n[:40]
+    m = re.search(r"gemm_kernel<(\d+), (\d+), \d+, \d+, 0, (9|10|11),", n)
+    return f"gemm_kernel {m[1]}x{m[2]} {GPT_PREFILL_GEMM[int(m[3])]}" if m else None
 
 
 def write_gpt_profiles(raw: Path, out: Path) -> None:
@@ -631,35 +637,30 @@ def write_gpt_profiles(raw: Path, out: Path) -> None:
     if not tr.exists() or not bt or "gpt_decode" not in bt:
         print(f"skip GPT tables: no {tr} / gpt_trace.log")
         return
-    rows = [r for r in load_trace(tr) if any(k in r["Kernel_Name"] for k in ("gemv", "attn_split", "attn_combine",
-                                                                              "sample_kernel", "embed", "argmax",
-                                                                              "advance_rows"))]
+    rows = load_trace(tr)
     roles = gemv_roles(rows, "Grid_Size_X", "Workgroup_Size_X")
     per = collections.defaultdict(list)
     for r in rows:
-        per[gpt_kernel_key(r, roles)].append(dur(r))
+        k = gpt_kernel_key(r, roles)
+        if k:
+            per[k].append(dur(r))
     body = [[f"`{k}`", len(v), f"{sum(v) / len(v):.2f}", f"{min(v):.2f}", f"{max(v):.2f}", f"{sum(v) / 1e3:.2f}"]
             for k, v in sorted(per.items(), key=lambda kv: -sum(kv[1]))]
     g = bt["gpt_decode"]
-    # the c_fc timing loop: the longest run of back-to-back c_fc GEMVs
-    best, i = (0, 0), 0
-    key_fc = next((k for k in per if k.startswith("gemv_kernel c_fc ")), None)
-    while i < len(rows):
-        if gpt_kernel_key(rows[i], roles) == key_fc:
-            j = i
-            while j < len(rows) and gpt_kernel_key(rows[j], roles) == key_fc:
-                j += 1
-            if j - i > best[1] - best[0]:
-                best = (i, j)
-            i = j
-        else:
-            i += 1
-    d = [dur(r) for r in rows[best[0]:best[1]]]
-    loop = f"average {sum(d) / len(d):.2f} us, min {min(d):.2f}, max {max(d):.2f}" if d else "not found"
+    fe = raw / "gptpmc_fetch" / "fetch_counter_collection.csv"
+    wr = raw / "gptpmc_write" / "write_counter_collection.csv"
+    sq = raw / "gptpmc_sq" / "sq_counter_collection.csv"
+    token = lambda r: "token_kernel" in r["Kernel_Name"]
+    counters = ""
+    if sq.exists():
+        mean = {c: (lambda v: sum(v) / max(len(v), 1))(pmc_per_dispatch(sq, c, token)) for c in GPT_SQ.split()}
+        counters = ("\n## Counters of `token_kernel` (mean of a dispatch)\n\n"
+                    + md_table(["counter", "value"], [[f"`{c}`", f"{v:,.0f}"] for c, v in mean.items()])
+                    + f"\n\nOf its waves' cycles {100 * mean['SQ_WAIT_ANY'] / max(mean['SQ_WAVE_CYCLES'], 1):.0f}% are waits.\n")
     cmds = "\n".join(GPT_CMDS)
     md = f"""# GPT mel-code decoder: 553 codes after a 150-row prefix, 24 layers -- rocprofv3 kernel trace
 
-Commands (repo root, MI355X, one GPU).  The HIP-graph replay is switched off with MIT2CFM_GRAPH=0, the resident step kernel with MIT2CFM_GPT_RESIDENT=0
+Commands (repo root, MI355X, one GPU).  The HIP-graph replay is switched off with MIT2CFM_GRAPH=0
 (every kernel launched directly; the same kernels): one earlier kernel-trace run with graph replay
 ended in a host SIGSEGV inside hipGraphLaunch of the GPT step graph.
 
@@ -668,44 +669,31 @@ ended in a host SIGSEGV inside hipGraphLaunch of the GPT step graph.
 ```
 
 bench.py `gpt_decode` of the traced run (direct launches, profiler attached): {g['ms_per_code']:.4f} ms per code, prefill
-{g['prefill_ms']:.3f} ms.  Without the profiler and with graph replay the bench's figure is the one in the round's bench line.
+{g['prefill_ms']:.3f} ms, {g['paths']['resident_steps']} token steps by `token_kernel` and {g['paths']['plain_steps']} by plain launches.
 
-## Per kernel (all dispatches of the GPT section; GEMVs named by product, with blocks x threads)
+## Per kernel (all dispatches of the GPT section; the GEMVs are the bench's loop of the plain launches' c_fc)
 
 {md_table(['kernel', 'dispatches', 'avg us', 'min us', 'max us', 'total ms'], body)}
-
-The roofline kernel's timing loop in this trace ({len(d)} back-to-back c_fc launches cycling the 24 layers'
-weights): {loop} (kernel execution from the trace timestamps).
-"""
+{counters}"""
     (out / "gpt_decode_P150_553codes_kernel_trace.md").write_text(md)
     print("wrote gpt_decode_P150_553codes_kernel_trace.md")
-    fe = raw / "gptpmc_fetch" / "fetch_counter_collection.csv"
-    wr = raw / "gptpmc_write" / "write_counter_collection.csv"
     cal = calibration(fe, wr)
     if cal:
-        def fc_match(path: Path, counter: str):
-            disp = {}
-            for r in csv.DictReader(open(path)):
-                if r["Counter_Name"] == counter:
-                    disp.setdefault(int(r["Dispatch_Id"]), r)
-            ordered = [disp[k] for k in sorted(disp)]
-            fc = [k for k, v in gemv_roles(ordered, "Grid_Size", "Workgroup_Size").items() if v == "c_fc"]
-            return lambda r: r["Kernel_Id"] in fc
-        f = pmc_per_dispatch(fe, "FETCH_SIZE", fc_match(fe, "FETCH_SIZE"))
-        w = pmc_per_dispatch(wr, "WRITE_SIZE", fc_match(wr, "WRITE_SIZE"))
+        f = pmc_per_dispatch(fe, "FETCH_SIZE", token)
+        w = pmc_per_dispatch(wr, "WRITE_SIZE", token)
         if f and w:
             fk, wk = sum(f) / len(f), sum(w) / len(w)
-            j = {"kernel": "gemv_gpt_c_fc",
-                 "workload": "GPT c_fc GEMV + LayerNorm prologue + gelu_new, 5120 x 1280 f16 weights, one 1280-wide input vector",
+            j = {"kernel": "token_kernel",
+                 "workload": "a GPT token step as one resident kernel: 24 layers, mel_head, 150 to 702 cached rows",
                  "fetch_size_kib_per_dispatch": round(fk, 1), "write_size_kib_per_dispatch": round(wk, 1),
                  "calibration": cal,
                  "hbm_bytes_per_launch": int(fk * cal["fetch_factor_bytes_per_kib"] + wk * cal["write_factor_bytes_per_kib"]),
-                 "algorithmic_bytes_per_launch": 5120 * 1280 * 2 + 1280 * 4 * 3 + 5120 * 4 * 2,
-                 "commands": GPT_CMDS[1:],
-                 "dispatches_used": f"every dispatch of the c_fc GEMV in the runs ({len(f)}); min/max FETCH_SIZE "
+                 "algorithmic_bytes_per_launch": g["roofline"]["algorithmic_bytes"],
+                 "commands": GPT_CMDS[1:3],
+                 "dispatches_used": f"every dispatch of the kernel in the runs ({len(f)}); min/max FETCH_SIZE "
                                     f"{min(f):.0f}/{max(f):.0f} KiB"}
-            (out / "traffic_gemv_gpt_c_fc.json").write_text(json.dumps(j, indent=1) + "\n")
-            print("wrote traffic_gemv_gpt_c_fc.json")
+            (out / "traffic_gpt_token_kernel.json").write_text(json.dumps(j, indent=1) + "\n")
+            print("wrote traffic_gpt_token_kernel.json")
 
 
 def unpack_raw(raw: Path) -> None:
