@@ -408,7 +408,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
 // alone it runs step after step, and another stream's kernels get only the gaps
 // between two of them (a mel decode of 128 frames took 158 ms beside a greedy
 // call instead of 6).  The kernel's workgroups start within 0.85 us of each other
-// on a free GPU (15,000 steps) and some microseconds apart where another kernel
+// on a free GPU (3,072 steps) and some microseconds apart where another kernel
 // holds CUs (more than 1.5 us in 85 to 95 of 100 steps), and that tells: two such
 // steps close together, as a single one comes up by itself now and then (one in
 // 1,000 under a profiler).  From then on, and for two steps after the last sign,

@@ -9,12 +9,11 @@
 // phase has just used, so about a layer's weights (39 MB over the chip) are
 // always in flight and no phase waits for HBM.
 //
-// What bounds it: the hand-overs, five a layer.  A code at 57 to 153 cached
-// rows takes 0.37 ms (15.2 us a layer) where the separate launches took 0.70;
-// 0.965 GB of weights and 4.8 TB/s would be 0.20.  Without the weight loads it
-// takes 0.35, so HBM is nearly hidden; a hand-over to all 256 workgroups takes
-// 0.9 us at best (of one word between two of them: 0.5), the LayerNorms,
-// splits and merges between them 5 us a layer, the products 1.2.
+// What bounds it: the hand-overs, five a layer.  A code takes 0.38 ms at 150
+// cached rows and 0.43 at 700 (15 us a layer), where the separate launches take
+// 0.65 and 0.71; 0.965 GB of weights at 4.8 TB/s would be 0.20.  Without the
+// weight loads it takes 0.33 at either, so HBM is nearly hidden; a hand-over to
+// all 256 workgroups takes 0.9 us at best (of one word between two of them: 0.5).
 //
 // Hand-over between workgroups.  A value that another workgroup needs is
 // stored as one 64-bit word, its tag (step and layer) above its bits, with a
@@ -71,7 +70,17 @@ constexpr int kSW = kW / 32 / kCW, kR3W = 448, kS3W = 2, kR3F = 1728, kS3F = 6, 
 static_assert(kSW * kCW * 32 == kW && kR4 == 32 * kCW, "whole steps per wave");
 static_assert(3 * kR3W >= kW && kS3W * kCW * 32 >= kR3W && 3 * kR3F >= kMLP && kS3F * kCW * 32 >= kR3F, "ranges");
 static_assert(kTokHeadRows <= 36, "the head's rows use the blocks of c_attn and c_fc");
-// Clocks / 64 that a phase's poll waits before its first look.
+// Clocks / 64 that a phase's poll waits before its first look: about as long as
+// its words take at best (poll says why).  ms a code at 20 / 150 / 400 / 700 /
+// 1,500 cached rows, all of them
+//   not at all       0.461 0.467 0.482 0.508 0.605
+//   x 0.5            0.404 0.412 0.432 0.450 0.547
+//   x 0.75           0.384 0.389 0.418 0.434 0.531
+//   as here          0.376 0.377 0.412 0.431 0.525
+//   x 1.25           0.382 0.382 0.408 0.430 0.523
+//   x 1.5            0.395 0.395 0.409 0.435 0.530
+//   the attention's (which takes longer with the rows) x 1.5, the others as here
+//                    0.386 0.385 0.404 0.432 0.526
 constexpr int kSleepXa = 56, kSleepQ = 4, kSleepAtt = 32, kSleepXb = 32, kSleepFc = 40;
 constexpr int kSleepIdle = 96;  // ... the attention's, more where a workgroup has no part in it
 
@@ -355,9 +364,9 @@ __device__ __forceinline__ void put_attention(const TokenArgs& a, Lds& s, int h,
 // ------------------------------------------------------------ product waves
 // A product is D = A B on the matrix cores: A's rows are weight rows (exact in
 // f16), B's columns 2 r and 2 r + 1 the hi and lo halves of the input over K
-// range r, so a row's value is D[row][2 r] + D[row][2 r + 1] / 2048.  (On the
-// vector units the conversions, products and lane sums of a phase took 1.2 us
-// of issue slots; so they take 0.2.)
+// range r, so a row's value is D[row][2 r] + D[row][2 r + 1] / 2048.  (As dot
+// products on the vector units, with their conversions and lane sums, a code
+// took 0.53 ms where it took 0.47 so, before the polls slept.)
 constexpr int kOob = 1 << 30;  // a byte offset past every buffer: reads zeros, without a memory access
 
 __device__ __forceinline__ half8 buffer_load8(buffer_rsrc_t r, int voffset) {
