@@ -201,8 +201,8 @@ def test_position_table_bound(ctx2, mit2):
 
 @pytest.mark.parametrize("P", [1, 7, 8, 9, 100])
 def test_chunked_prefill_equals_row_prefill(ctx2, monkeypatch, P):
-    """The prefill's chunks of 8 rows give the values of prefilling one row at a
-    time through the decode step's kernels (same sums in the same order)."""
+    """The prefix taken as row products gives the values of prefilling one row at a
+    time through the plain step's kernels, to fp32 rounding."""
     prefix = _prefix(P, seed=20 + P)
     chunked = ctx2.gpt_kv_greedy(prefix, 4)
     monkeypatch.setenv("MIT2CFM_GPT_ROW_PREFILL", "1")
