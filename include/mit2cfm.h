@@ -495,7 +495,7 @@ mit2cfm_status mit2cfm_gpt_cached_decode(mit2cfm_ctx* ctx, const float* rows, ui
  * throughout, take over where a value does not fit such a pair and where the
  * resident kernel cannot have the GPU (its results are the same to fp32
  * rounding).  A wait runs out when other work, as another process's resident
- * kernel, holds some of the GPU for about a second: the rest of that call is
+ * kernel, holds some of the GPU for about 25 ms: the rest of that call is
  * plain, and so are the context's next 1, 2, 4 .. 64 calls while it goes on. */
 typedef struct mit2cfm_gpt_counts {
   uint64_t resident_steps; /* token steps by the resident kernel */

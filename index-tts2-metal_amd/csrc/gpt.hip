@@ -1272,13 +1272,17 @@ struct GptDecoder::Impl {
   GptDecoder::Counts counts;
   // The resident step kernel decodes tokens (else the separate launches do):
   // all its workgroups fit the device.  A call in which a wait of it ran out (a
-  // neighbour kept some of the CUs for about a second) leaves the next calls
+  // neighbour kept some of the CUs for about 25 ms) leaves the next calls
   // plain: 1, then 2, 4 .. kMostSkipped of them while that goes on, as each try
   // costs the wait; 1 again after a call that ran through.
   bool resident = false;
   static constexpr int kMostSkipped = 64;
   int skip_calls = 0, next_skip = 1;
-  uint32_t spin_limit = 1u << 20;  // env MIT2CFM_GPT_SPIN_LIMIT (for checking: 1 gives up at once)
+  // Polls a wait may take, about 25 ms: past any one kernel of this library (0.4
+  // ms) by far, and short for what it is there for, two processes whose resident
+  // kernels each hold CUs the other needs.  Two such processes, 256 codes a call:
+  // 229 to 316 ms (a million polls: up to 461; plain launches alone: 262).
+  uint32_t spin_limit = 1u << 17;  // env MIT2CFM_GPT_SPIN_LIMIT (for checking: 1 gives up at once)
   size_t layer_stride = 0;  // bytes from a layer's arrays to the next's
   bool use_graph = true;  // env MIT2CFM_GRAPH=0: launch every kernel directly (for profilers)
   // The measurement hook's launch loop, captured once per (kernel, count)

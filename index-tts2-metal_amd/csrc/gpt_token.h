@@ -40,7 +40,7 @@ struct TokenArgs {
   float* blk_val;  // [kTokWG] first maximum of each workgroup's logits and its row
   int* blk_idx;
   uint32_t* start;  // [kTokWG] when each workgroup started (device_ticks)
-  uint32_t spin_limit;  // polls a wait may take (a million: about a second)
+  uint32_t spin_limit;  // polls a wait may take (0.2 us each)
 };
 
 // The device's constant clock: ticks of 10 ns.
