@@ -412,19 +412,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(GemvArgs a) {
 // holds CUs (more than 1.5 us in 85 to 95 of 100 steps), and that tells: two such
 // steps close together, as a single one comes up by itself now and then (one in
 // 1,000 under a profiler).  From then on, and for two steps after the last sign,
-// each step owes the others twice its time, and once 2.3 ms are owed the pick
-// behind a step waits them off: its one CU apart the GPU is free.  Beside it
-// (256 codes after 150 rows, alone 104 ms; plain launches, which share the GPU by
-// themselves, in brackets):
-//   mel decode, 860 frames   greedy 307 ms [317]  a decode 35.5 ms [31.7], alone 21.6
-//   mel decode, 128 frames          304 [265]              9.9 [9.6], 6.0
-//   vocoder, 861 frames             348 [437]              9.0 [7.7], 6.2
-//   condition, 553 codes            303 [255]              0.15 [0.13], 0.10
-// (2.5 times: 358 and 33.6 in the first row; waits after every step: 311 and 38.8,
-// as the others then refill the caches each time).
+// each step owes the others 1.75 times its time, more (up to 3.5 times) where the
+// starts lie 10 to 20 us apart, as kernels that long keep the GPU full by
+// themselves, and once 2.3 ms are owed the pick behind a step waits them off: its
+// one CU apart the GPU is free.  Beside it, in ms (256 codes after 150 rows, alone
+// 104; in brackets the plain launches, which share the GPU by themselves):
+//   mel decode, 860 frames     greedy 300 [317]  a decode 36.1 [31.7], alone 21.6
+//   mel decode, 128 frames            293 [265]           10.2 [9.6], 6.0
+//   mel decode, 3,000 frames          372 [462]            102 [77], 63
+//   mel batch, 8 requests             419 [556]            157 [119], 102
+//   vocoder, 861 frames               461 [437]            8.0 [7.7], 6.2
+//   condition, 553 codes              283 [255]           0.15 [0.13], 0.10
+// (twice throughout: 348 and 8.9 for the vocoder, 343 and 171 for the batch; 2.5
+// times: 358 and 33.6 in the first row; waits after every step: 311 and 38.8, as
+// the others then refill the caches each time.)  A kernel too short to be seen
+// waits for the step that runs: 0.26 ms for a 0.02 ms one.
 constexpr int kYieldSpread = 150;                 // ticks of 10 ns
 constexpr int kYieldSign = 3, kYieldFull = 6;     // a sign's weight, which a step without one lowers by 1
-constexpr uint32_t kYieldShare = 2, kYieldLeast = 230000, kYieldMost = 800000;
+constexpr uint32_t kYieldLong = 1000, kYieldLeast = 230000, kYieldMost = 800000;
 constexpr int kYieldLooks = 20000;  // bound of the wait, about 1 us each
 constexpr int kYieldWave = 15;      // of the pick kernels' 16
 // The yield wave's share of the workgroups' start times, read ahead.
@@ -455,8 +460,13 @@ __device__ __forceinline__ void yield_gpu(GptState* st, const uint32_t* start, c
   }
   const uint32_t now = device_ticks(), took = now - t0 - (uint32_t)first;
   int signs = st->yield_signs;
-  signs = last - first > kYieldSpread ? min(signs + kYieldSign, kYieldFull) : max(signs - 1, 0);
-  uint32_t owed = signs > kYieldSign ? min(st->owed + took * kYieldShare, kYieldMost) : 0u;
+  const uint32_t spread = (uint32_t)(last - first);
+  signs = spread > kYieldSpread ? min(signs + kYieldSign, kYieldFull) : max(signs - 1, 0);
+  uint32_t owed = 0;
+  if (signs > kYieldSign) {
+    const uint32_t longer = min(max(spread, kYieldLong) - kYieldLong, kYieldLong);
+    owed = min(st->owed + took * 7 / 4 + took * longer / (kYieldLong * 4 / 7), kYieldMost);
+  }
   const bool now_due = owed >= kYieldLeast;
   if ((threadIdx.x & 63) == 0) {
     st->yield_signs = signs;
